@@ -106,6 +106,25 @@ def test_decode_many_splits_merge(cuda, monkeypatch):
     check(_with_lengths(case, lens, cuda), range(8), TOL_BF16)
 
 
+@pytest.mark.parametrize("d", [128, 256])
+@pytest.mark.parametrize("streamk", ["0", "1"])
+def test_decode_merge_groups(cuda, d, streamk, monkeypatch):
+    """Few sequences with hundreds of pieces per head: the merge's 8 thread
+    groups take 8 pieces each per round (64 in all), so rows of 1, 2, 8, 9,
+    64, 65 and 71 splits (stream-K at head_dim 256: 32-token ranges) end
+    inside, at and past a group's chunk and the round."""
+    monkeypatch.setenv("NQ_DECODE_SPLIT_TOKENS", "128")
+    monkeypatch.setenv("NQ_DECODE_STREAMK", streamk)
+    case = make_decode_case("cfg2", seed=21, device=cuda, batch=8, ctx=(1, 1), hq=4096 // d, hkv=1024 // d, d=d)
+    lens = torch.tensor([0, 128, 129, 1024, 1025, 8192, 8193, 9000], dtype=torch.int32)
+    case = _with_lengths(case, lens, cuda)
+    for name in ("k_cache", "v_cache"):
+        case[name] = case[name].view(-1, 256, 1024 // d, d)
+    case["slot_mapping"][0] = -1
+    check(case, range(1, 8), TOL_BF16)
+    assert torch.all(case["_out"][0] == 0)
+
+
 def test_decode_ctx1_returns_new_value(cuda):
     case = make_decode_case("cfg2", seed=5, device=cuda, batch=4, ctx=(1, 1))
     out = run_step(case)
