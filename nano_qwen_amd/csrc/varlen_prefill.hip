@@ -69,6 +69,7 @@ struct PrefillArgs {
   int pin;          // work groups pinned to XCDs (>= 8 groups)
   int by_cost;      // persistent kernel: 0 query-tile order; cost order over live items (num_seqs <= kMaxSeqs),
                     // 1 each item derived when taken, 2 read from a list built at launch
+  int rep_log2;     // 2^rep_log2 XCDs share each kv-head slot, every 2^rep_log2-th query tile each (by_cost == 2)
   int level_shift;  // cost level of an item: its key tiles >> level_shift (< n_levels)
   int n_levels;
   const uint8_t *gate;  // null, or Qwen3.5's output gate [total_q, Hq, D] (type of out)
@@ -233,10 +234,19 @@ struct CostQueue {
   const uint32_t *tab;  // LDS: the queue's items in order (by_cost == 2)
   int x, n_y, rows, ystep;
   int rows_log2, ystep_log2;  // rows and ystep are powers of two
+  int rep_log2, r;            // the queue holds query tiles r, r + 2^rep_log2, ... (all of them when 0)
 };
 // Kv-head slots of sequence s in the queue: y0, y0 + ystep, ... < n_y.
 __device__ __forceinline__ int first_slot(const CostQueue &cq, int s) {
+  if (cq.rep_log2 > 0) return cq.x & (cq.n_y - 1);
   return cq.ystep == 8 ? ((cq.x - s * cq.n_y) & 7) : 0;
+}
+// Query tiles below n that the queue holds.
+__device__ __forceinline__ int own_tiles(const CostQueue &cq, int n) {
+  return (n + (1 << cq.rep_log2) - 1 - cq.r) >> cq.rep_log2;
+}
+__device__ __forceinline__ bool own_tile(const CostQueue &cq, int qt) {
+  return (qt & ((1 << cq.rep_log2) - 1)) == cq.r;
 }
 __device__ __forceinline__ int n_slots(const CostQueue &cq, int y0) {
   return y0 < cq.n_y ? ((cq.n_y - 1 - y0) >> cq.ystep_log2) + 1 : 0;
@@ -412,7 +422,7 @@ __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
   uint32_t *ctr = a.queue + x;
   const int item_rows = 16 * QS * (NW / a.G4);
   const CostQueue cq{lds_lev, lds_cuq,   lds_cuk, lds_tab, x, n_y, item_rows, a.pin ? 8 : 1, 31 - __builtin_clz(item_rows),
-                     a.pin ? 3 : 0};
+                     a.pin ? 3 : 0, a.rep_log2, a.rep_log2 > 0 ? x / n_y : 0};
   if (a.by_cost) {
     // Sequence bounds into LDS, then the live items of this queue counted
     // per cost level, then each level's first index (highest level first).
@@ -426,7 +436,7 @@ __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
       const int sq = i / n_x, qt = i - sq * n_x;
       const int Lq = lds_cuq[sq + 1] - lds_cuq[sq];
       const int w = n_slots(cq, first_slot(cq, sq));
-      if (qt * cq.rows < Lq && w > 0)
+      if (qt * cq.rows < Lq && w > 0 && own_tile(cq, qt))
         atomicAdd(&lds_lev[cost_level(a, cq, qt, Lq, lds_cuk[sq + 1] - lds_cuk[sq])], w);
     }
     __syncthreads();
@@ -460,7 +470,7 @@ __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
             const int nq = Lq > 0 ? (Lq + cq.rows - 1) >> cq.rows_log2 : 0;
             const int qlo = first_tile_with(a, cq, lo_v, nq, Lk, Lk - Lq);
             const int qhi = L == a.n_levels - 1 ? nq : first_tile_with(a, cq, hi_v, nq, Lk, Lk - Lq);
-            cnt = max(0, qhi - qlo) * n_slots(cq, first_slot(cq, s));
+            cnt = max(0, own_tiles(cq, qhi) - own_tiles(cq, qlo)) * n_slots(cq, first_slot(cq, s));
           }
           const int incl = wave_iscan(cnt);
           if (s < a.num_seqs) first[L * a.num_seqs + s] = carry + incl - cnt;
@@ -472,13 +482,14 @@ __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
         const int sq = i / n_x, qt = i - sq * n_x;
         const int Lq = lds_cuq[sq + 1] - lds_cuq[sq], Lk = lds_cuk[sq + 1] - lds_cuk[sq];
         const int y0 = first_slot(cq, sq), w = n_slots(cq, y0);
-        if (qt * cq.rows < Lq && w > 0) {
+        if (qt * cq.rows < Lq && w > 0 && own_tile(cq, qt)) {
           const int L = cost_level(a, cq, qt, Lq, Lk);
           const int nq = (Lq + cq.rows - 1) >> cq.rows_log2;
           const int qlo = first_tile_with(a, cq, L << a.level_shift, nq, Lk, Lk - Lq);
           const int qhi = L == a.n_levels - 1 ? nq : first_tile_with(a, cq, (L + 1) << a.level_shift, nq, Lk, Lk - Lq);
-          int pos = first[L * a.num_seqs + sq] + (qhi - 1 - qt);
-          for (int yi = 0; yi < w; ++yi, pos += qhi - qlo)
+          const int nt = own_tiles(cq, qhi);
+          int pos = first[L * a.num_seqs + sq] + nt - 1 - own_tiles(cq, qt);
+          for (int yi = 0; yi < w; ++yi, pos += nt - own_tiles(cq, qlo))
             lds_tab[pos] = (static_cast<uint32_t>(sq) << 22) | (static_cast<uint32_t>(y0 + cq.ystep * yi) << 14) | qt;
         }
       }
@@ -1273,7 +1284,7 @@ int launch_prefill_dma(PrefillArgs a, hipStream_t st) {
   const int rows_per_item = S::ITEM_ROWS / a.G4;
   a.n_qtiles = (a.max_seqlen_q + rows_per_item - 1) / rows_per_item;
   const int64_t U = static_cast<int64_t>(a.Hkv) * a.quads * a.num_seqs;
-  const int64_t total = work_grid(a.n_qtiles, U);
+  int64_t total = work_grid(a.n_qtiles, U);
   if (total > 0x7fffffff) return fail(NQ_EINVAL, "varlen_prefill: too many work items");
   if (!a.queue) return fail(NQ_EINVAL, "varlen_prefill: null workspace");
   a.pin = U >= 8;
@@ -1288,9 +1299,27 @@ int launch_prefill_dma(PrefillArgs a, hipStream_t st) {
   // (its groups x query tiles bound it), the (level, sequence) starts fit the
   // ring and the packed words hold the fields.
   const int64_t cx_max = U >= 8 ? (U + 7) / 8 : U;
-  if (a.by_cost && cx_max * a.n_qtiles <= S::MAX_ITEMS && static_cast<int64_t>(a.num_seqs) * a.n_levels * 4 <= S::RING_BYTES &&
+  // Fewer than 8 kv-head slots that divide 8: each slot belongs to 8 / n_y
+  // XCDs, which take its query tiles in turn, so that every XCD carries the
+  // same work whatever the lengths (with groups pinned whole, 4 slots put the
+  // even sequences on one half of the XCDs and the odd ones on the other:
+  // 6 prompts of 333-2567 tokens, 4 kv heads of 256, 349 -> 255 us; 16 prompts
+  // of 256-2048 behind prefixes, 4 kv heads of 128, 215 -> 178 us).  A slot's
+  // K/V is then read into 2, 4 or 8 L2s instead of one.
+  const int n_y = a.Hkv * a.quads;
+  int rep_log2 = 0;
+  while (n_y << rep_log2 < 8) ++rep_log2;
+  if (n_y << rep_log2 == 8 && rep_log2 > 0 &&
+      static_cast<int64_t>(a.num_seqs) * ((a.n_qtiles + (1 << rep_log2) - 1) >> rep_log2) <= S::MAX_ITEMS)
+    a.rep_log2 = rep_log2;
+  if (a.by_cost && (a.rep_log2 > 0 || cx_max * a.n_qtiles <= S::MAX_ITEMS) && static_cast<int64_t>(a.num_seqs) * a.n_levels * 4 <= S::RING_BYTES &&
       U / a.num_seqs <= 256 && a.n_qtiles <= 16384)
     a.by_cost = 2;
+  if (a.by_cost != 2) a.rep_log2 = 0;
+  if (a.rep_log2 > 0) {
+    a.pin = 1;
+    total = 8 * static_cast<int64_t>(a.num_seqs) * ((a.n_qtiles + (1 << a.rep_log2) - 1) >> a.rep_log2);
+  }
   // S::WG_PER_CU resident workgroups per CU, never more than there are
   // items; a multiple of 8 so every XCD gets the same count.
   int64_t grid = (static_cast<int64_t>(device_cus()) * S::WG_PER_CU + 7) / 8 * 8;
