@@ -307,6 +307,40 @@ int nq_varlen_prefill_gated(const void *q, int64_t q_row_stride, int64_t q_head_
                             const void *gate, int64_t gate_row_stride, int64_t gate_head_stride,
                             int64_t total_q, void *stream);
 
+/*
+ * nq_varlen_prefill (or, with a gate, nq_varlen_prefill_gated) with room for
+ * partial outputs, for launches with too few work items to share evenly (a
+ * short prompt, a few new tokens behind long prefixes): each queue's key tiles
+ * are cut into one equal range per workgroup, and a second kernel merges the
+ * float32 partial outputs of the items that a cut crosses.  Launches with
+ * enough items, or whose split_workspace is null or smaller than
+ * nq_prefill_split_workspace_bytes, run as the two calls above; gate may be
+ * null.  total_q: rows of q (the items are bounded from it).  split_workspace
+ * must be 256-byte aligned; its contents need no clearing.  Calls that overlap
+ * may not share one.
+ */
+int nq_varlen_prefill_split(const void *q, int64_t q_row_stride, int64_t q_head_stride,
+                            const void *k, const void *v, int64_t kv_row_stride,
+                            const int32_t *cu_seqlens_q, const int32_t *cu_seqlens_k,
+                            int max_seqlen_q, int max_seqlen_k,
+                            const int32_t *block_tables, int64_t bt_stride,
+                            int max_blocks_per_seq, int64_t num_blocks,
+                            void *out, int64_t out_row_stride, int64_t out_head_stride,
+                            int num_seqs, int num_q_heads, int num_kv_heads,
+                            int head_dim, int block_size, float softmax_scale,
+                            int causal, int q_dtype, int kv_dtype,
+                            const float *k_scale, const float *v_scale,
+                            void *workspace, int64_t workspace_bytes,
+                            const void *gate, int64_t gate_row_stride, int64_t gate_head_stride,
+                            int64_t total_q, void *split_workspace, int64_t split_workspace_bytes,
+                            void *stream);
+
+/* Bytes of split_workspace with which nq_varlen_prefill_split cuts a launch of
+ * these sizes into equal ranges; 0: it would not (decided from the sizes and
+ * the current device alone). */
+int64_t nq_prefill_split_workspace_bytes(int num_seqs, int64_t total_q, int max_seqlen_q, int max_seqlen_k,
+                                         int num_q_heads, int num_kv_heads, int head_dim);
+
 /* Bytes of device workspace nq_varlen_prefill needs (work-queue counters). */
 int64_t nq_prefill_workspace_bytes(void);
 

@@ -62,6 +62,12 @@ _SIGS = {
                                         c_int, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64,
                                         c_int64, c_int64, c_void_p]),
     "nq_prefill_workspace_bytes": (c_int64, []),
+    "nq_varlen_prefill_split": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_void_p,
+                                        c_void_p, c_int, c_int, c_void_p, c_int64, c_int, c_int64, c_void_p,
+                                        c_int64, c_int64, c_int, c_int, c_int, c_int, c_int, c_float, c_int,
+                                        c_int, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64,
+                                        c_int64, c_int64, c_void_p, c_int64, c_void_p]),
+    "nq_prefill_split_workspace_bytes": (c_int64, [c_int, c_int64, c_int, c_int, c_int, c_int, c_int]),
     "nq_prepare_decode": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                   c_void_p, c_int, c_int, c_void_p]),
     "nq_gdn_decode": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64,

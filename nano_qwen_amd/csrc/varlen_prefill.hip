@@ -29,6 +29,7 @@
 //    operand reads are bank-conflict free.
 //  * Online softmax in the log2 domain with lazy rescaling: O and l are only
 //    rescaled when a row maximum grows by more than 2^8, so P <= 256.
+#include <algorithm>
 #include <type_traits>
 
 #include "nq_device.hpp"
@@ -74,7 +75,13 @@ struct PrefillArgs {
   int n_levels;
   const uint8_t *gate;  // null, or Qwen3.5's output gate [total_q, Hq, D] (type of out)
   int64_t g_rs, g_hs;   // bytes
+  // Equal ranges (kMode 2): partial outputs of range slot i (fp32, normalised,
+  // in the order the waves hold them), their log2-sum-exp, and what they are.
+  float *part_o;
+  float *part_l;
+  int4 *part_desc;  // (sequence, first head, first row, piece: kPieceNone / kPieceMore / kPieceLast)
 };
+constexpr int kPieceNone = -1, kPieceMore = 0, kPieceLast = 1;
 
 // Chunk swizzles of the 16-bit DMA kernel's LDS tiles (16-byte chunk c of
 // key row r is stored at chunk c ^ swz(r)), one per tile because the two
@@ -106,6 +113,19 @@ __device__ inline int swz8(int row) {
 // however the lengths vary.  Fewer than 8 groups: no pinning.
 // Work items of the queues: n_x query tiles of each group, 8 equal queues
 // when pinned.
+// log2 of the XCDs that share each kv-head slot when there are fewer than 8
+// slots and their number divides 8 (0 otherwise): those XCDs take the slot's
+// query tiles in turn, so that every XCD carries the same work whatever the
+// lengths.  With groups pinned whole, 4 slots put the even sequences on one
+// half of the XCDs and the odd ones on the other: 6 prompts of 333-2567
+// tokens, 4 kv heads of 256, 349 -> 255 us; 16 prompts of 256-2048 behind
+// prefixes, 4 kv heads of 128, 215 -> 178 us.  A slot's K/V is then read into
+// 2, 4 or 8 L2s instead of one.
+inline int shared_slots_log2(int n_y) {
+  int l = 0;
+  while (n_y << l < 8) ++l;
+  return n_y << l == 8 ? l : 0;
+}
 inline int64_t work_grid(int64_t n_x, int64_t U) { return U >= 8 ? 8 * ((U + 7) / 8) * n_x : U * n_x; }
 
 // 16-bit K/V: persistent workgroups fed by an LDS DMA ring.
@@ -167,6 +187,10 @@ using ShapeD = PShape<8, 1, 2, 4, 256>;
 struct Item {
   bool live;
   int s, kvh, head0, q0, Lq, k0, Lk, P, row_begin, key_end, n_kt;
+  // Equal ranges only: the first block-table entry of its keys (k0, Lk, P and
+  // key_end then count from its first key), its partial-output slot (-1: the
+  // item is whole) and whether it holds the item's last key tiles.
+  int blk0, part, last;
 };
 
 // Item fields of query tile qt of kv-head slot y of sequence s.
@@ -337,6 +361,95 @@ __device__ __forceinline__ Item describe_by_table(const PrefillArgs &a, const Co
   return fill_item(a, s, y, qt, cq.rows, q0, cq.cuq[s + 1] - q0, k0, cq.cuk[s + 1] - k0);
 }
 
+// Equal ranges (kMode 2), for launches with fewer items than the resident
+// workgroups can share evenly: each queue's live items laid end to end, each
+// as its key tiles + kRangeItem tiles of fixed cost, are cut into one equal
+// range per workgroup.  A workgroup's range covers whole items and at most
+// two partial ones (slot 2w: an item begun in an earlier range, slot 2w + 1:
+// one that continues in the next range); prefill_merge_kernel combines the
+// pieces of each cut item.  cum[e]: cost before entry e, where entry
+// (sequence, own query tile, kv-head slot) is e = (s * n_own + k) * w + yi and
+// entries without rows cost nothing.
+//
+// A launch with one item per workgroup or fewer lasts as long as its longest
+// item, on a chip that is mostly idle.  Measured, store included, whole items
+// against ranges: one prompt of 1111 tokens, 8 kv heads of 128 (280 items of
+// 1-35 key tiles on 512 workgroups) 72 -> 47.5 us; four prompts of 104-232
+// tokens behind 4352-5632 cached fp8 ones (200 items of 140-184 tiles) 304 ->
+// 105; one of 4000 tokens 215 -> 170; one of 2000 at 4 kv heads of 256 140 ->
+// 80.5.  What is left beside the tiles: the partial outputs (about 700 of 64
+// KiB, written and read once: 12-15 us of merge at 4-5 TB/s).
+// With 6 (12) tiles for an item's fixed cost: 0-5% (0-2%) slower; pieces of at
+// least 6 (10) tiles: 3-10% (5-20%) slower.
+constexpr int kRangeItem = 8;  // fixed cost of an item in key tiles (its transition, about 7 us)
+constexpr int kRangeKeys = 512;  // launches whose longest sequence has fewer keys run whole items
+constexpr int kRangeWaves = 2;   // launches with more items per resident workgroup than this, too
+constexpr int kRangeMin = 2;   // key tiles of a piece: shorter ones go to the neighbouring range
+struct Ranges {
+  const int *cum;  // LDS
+  int n, n_own, w, gran;  // entries, own query tiles, slots per sequence, key tiles a cut is a multiple of
+  int pos, end;           // this workgroup's range, the part not yet taken
+  int lin;                // its index among all ranges
+};
+// Entry with cum[e] <= c < cum[e + 1].  Called by whole waves.
+__device__ __forceinline__ int range_find(const Ranges &rg, int c) {
+  const int lane = threadIdx.x & 63;
+  const int step = (rg.n + 63) / 64;
+  const int i = min(lane * step, rg.n - 1);
+  const int b = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane * step < rg.n && rg.cum[i] <= c)) - 1;
+  const int base = b * step;
+  const int i2 = min(base + lane, rg.n - 1);
+  const int k = __builtin_popcountll(
+      __builtin_amdgcn_ballot_w64(lane < step && base + lane < rg.n && rg.cum[i2] <= c));
+  return __builtin_amdgcn_readfirstlane(base + k - 1);
+}
+// Key tile of an item of n_kt where a cut at cost x falls.
+__device__ __forceinline__ int range_tile(const Ranges &rg, int x, int n_kt) {
+  const int t = small_div(max(0, x - kRangeItem) + rg.gran / 2, rg.gran) * rg.gran;
+  return t < kRangeMin ? 0 : (t > n_kt - kRangeMin ? n_kt : t);
+}
+// The next piece of this workgroup's range (not live past its end).
+__device__ __forceinline__ Item range_next(const PrefillArgs &a, const CostQueue &cq, Ranges &rg, int key_tiles_per_blk) {
+  Item it{};
+  it.live = false;
+  while (rg.pos < rg.end) {
+    const int e = range_find(rg, rg.pos);
+    const int lo = __builtin_amdgcn_readfirstlane(rg.cum[e]), hi = __builtin_amdgcn_readfirstlane(rg.cum[e + 1]);
+    const int x0 = rg.pos - lo;
+    const bool cut = hi > rg.end;
+    const int x1 = rg.end - lo;
+    rg.pos = cut ? rg.end : hi;
+    const int sk = small_div(e, rg.w), yi = e - sk * rg.w;
+    const int s = small_div(sk, rg.n_own), k = sk - s * rg.n_own;
+    const int q0 = cq.cuq[s], k0 = cq.cuk[s];
+    it = fill_item(a, s, first_slot(cq, s) + cq.ystep * yi, (k << cq.rep_log2) + cq.r, cq.rows, q0, cq.cuq[s + 1] - q0,
+                   k0, cq.cuk[s + 1] - k0);
+    it.part = -1;
+    it.last = 1;
+    if (it.n_kt == 0) {  // a row without keys: its zeros belong to the range it begins in
+      if (x0 == 0) return it;
+      continue;
+    }
+    const int t0 = x0 > 0 ? range_tile(rg, x0, it.n_kt) : 0;
+    const int t1 = cut ? range_tile(rg, x1, it.n_kt) : it.n_kt;
+    if (t1 <= t0) continue;
+    if (t0 > 0 || t1 < it.n_kt) {
+      it.part = 2 * rg.lin + (t0 > 0 ? 0 : 1);
+      it.last = t1 == it.n_kt;
+      const int key0 = t0 * kKeys;
+      it.k0 += key0;
+      it.Lk -= key0;
+      it.P -= key0;
+      it.key_end = (it.last ? it.key_end : t1 * kKeys) - key0;
+      it.n_kt = t1 - t0;
+      it.blk0 = small_div(t0, key_tiles_per_blk);
+    }
+    return it;
+  }
+  it.live = false;
+  return it;
+}
+
 // Persistent prefill: S::WG_PER_CU workgroups per CU pull work items from
 // per-XCD queues.  The hardware dispatcher keeps only about half of the CUs
 // busy when one-per-CU workgroups of very different lengths are launched as
@@ -371,9 +484,10 @@ __device__ __forceinline__ Item describe_by_table(const PrefillArgs &a, const Co
 // waits count only younger stream entries -- except that a new item's first
 // kAhead tiles may precede the Q loads and the previous item's output stores
 // (a fixed count per wave), which the waits then add.
-template <class T, int D, class S, bool GATED, bool FP8, bool TAB>
+template <class T, int D, class S, bool GATED, bool FP8, int MODE>
 __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
   using DT = DTile<T, D>;
+  constexpr bool TAB = MODE == 1, RANGES = MODE == 2;
   constexpr int NW = S::NW, QS = S::QS, kSlots = S::SLOTS, kAhead = S::AHEAD;
   constexpr int RW = 16 * QS;        // query rows per wave
   constexpr int CR = kKeys / NW;     // tile rows each wave copies
@@ -423,7 +537,59 @@ __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
   const int item_rows = 16 * QS * (NW / a.G4);
   const CostQueue cq{lds_lev, lds_cuq,   lds_cuk, lds_tab, x, n_y, item_rows, a.pin ? 8 : 1, 31 - __builtin_clz(item_rows),
                      a.pin ? 3 : 0, a.rep_log2, a.rep_log2 > 0 ? x / n_y : 0};
-  if (a.by_cost) {
+  [[maybe_unused]] Ranges rg{};
+  if constexpr (RANGES) {
+    int *cum = reinterpret_cast<int *>(lds_tab);
+    for (int i = threadIdx.x; i <= a.num_seqs; i += blockDim.x) {
+      lds_cuq[i] = a.cu_q[i];
+      lds_cuk[i] = a.cu_k[i];
+    }
+    __syncthreads();
+    rg.cum = cum;
+    rg.n_own = own_tiles(cq, n_x);
+    rg.w = cq.rep_log2 > 0 ? 1 : (a.pin ? (n_y + 7) >> 3 : n_y);
+    rg.n = a.num_seqs * rg.n_own * rg.w;
+    const int tpb = paged ? a.block_size / kKeys : 1;
+    rg.gran = tpb >= 4 ? tpb : tpb * ((3 + tpb) / tpb);
+    // Exclusive prefix sums of the costs: each thread a run of entries.
+    const int per = (rg.n + 64 * NW - 1) / (64 * NW), e0 = min(static_cast<int>(threadIdx.x) * per, rg.n);
+    const int e1 = min(e0 + per, rg.n);
+    auto cost = [&](int e) {
+      const int sk = small_div(e, rg.w), yi = e - sk * rg.w;
+      const int s = small_div(sk, rg.n_own), k = sk - s * rg.n_own;
+      const int Lq = lds_cuq[s + 1] - lds_cuq[s], Lk = lds_cuk[s + 1] - lds_cuk[s];
+      const int row0 = ((k << cq.rep_log2) + cq.r) * cq.rows;
+      if (row0 >= Lq || yi >= n_slots(cq, first_slot(cq, s))) return 0;
+      const int key_end = a.causal ? max(0, min(Lk, min(row0 + cq.rows, Lq) + Lk - Lq)) : Lk;
+      return (key_end + kKeys - 1) / kKeys + kRangeItem;
+    };
+    int sum = 0;
+    for (int e = e0; e < e1; ++e) sum += cost(e);
+    const int incl = wave_iscan(sum);
+    if (lane == 63) lds_item[wave] = incl;  // 8 words: the item slots and the queue size
+    __syncthreads();
+    int run = incl - sum;
+    for (int i = 0; i < wave; ++i) run += lds_item[i];
+    for (int e = e0; e < e1; ++e) {
+      cum[e] = run;
+      run += cost(e);
+    }
+    if (threadIdx.x == 64 * NW - 1) cum[rg.n] = run;
+    __syncthreads();
+    const int total = __builtin_amdgcn_readfirstlane(cum[rg.n]);
+    // One range per workgroup of the queue, fewer when they would be shorter
+    // than a piece.
+    const int n_wg = a.pin ? static_cast<int>(gridDim.x) >> 3 : static_cast<int>(gridDim.x);
+    const int w = a.pin ? static_cast<int>(blockIdx.x) >> 3 : static_cast<int>(blockIdx.x);
+    const int n_rg = max(1, min(n_wg, total / (2 * kRangeMin + kRangeItem)));
+    rg.lin = (a.pin ? x * n_wg : 0) + w;
+    rg.pos = w < n_rg ? static_cast<int>(static_cast<int64_t>(w) * total / n_rg) : 0;
+    rg.end = w < n_rg ? static_cast<int>(static_cast<int64_t>(w + 1) * total / n_rg) : 0;
+    rg.pos = __builtin_amdgcn_readfirstlane(rg.pos);
+    rg.end = __builtin_amdgcn_readfirstlane(rg.end);
+    if (threadIdx.x < 2) a.part_desc[2 * rg.lin + threadIdx.x] = int4{0, 0, 0, kPieceNone};
+    __syncthreads();  // the descriptors are overwritten by the pieces below (thread 0)
+  } else if (a.by_cost) {
     // Sequence bounds into LDS, then the live items of this queue counted
     // per cost level, then each level's first index (highest level first).
     for (int i = threadIdx.x; i <= a.num_seqs; i += blockDim.x) {
@@ -530,6 +696,7 @@ __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
   int nx_head = 0;      // its kv head's byte offset within a row
   int64_t nx_base = 0;  // paged: address of its block-table row; packed: byte offset of its first key
   int nx_blk0 = 0;      // paged: its first block-table entry
+  int nx_bidx = 0;      // paged: and that entry's index
   int nx_first = 0;     // stream index of the queued item's first tile, once started
   // A copied tile lay in a missing block: from then on every tile takes the
   // masked path (which checks its block); plain_end bounds the current
@@ -560,7 +727,8 @@ __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
     if (paged) {
       const int32_t *bt = a.block_tables + static_cast<int64_t>(it.s) * a.bt_stride;
       nx_base = static_cast<int64_t>(reinterpret_cast<uintptr_t>(bt));
-      nx_blk0 = nx_rem > 0 ? blk_entry(bt, 0) : 0;
+      nx_bidx = RANGES ? it.blk0 : 0;
+      nx_blk0 = nx_rem > 0 ? blk_entry(bt, nx_bidx) : 0;
     } else {
       nx_base = static_cast<int64_t>(it.k0) * kv_rs + nx_head;
     }
@@ -574,7 +742,7 @@ __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
       st_bt = paged ? reinterpret_cast<const int32_t *>(static_cast<uintptr_t>(nx_base)) : nullptr;
       st_src = kbase + (paged ? 0 : nx_base);
       st_blk_next = nx_blk0;
-      st_bidx = 0;
+      st_bidx = RANGES ? nx_bidx : 0;
       st_left = paged ? 0 : 0x40000000;
       nx_first = st_pos;
     }
@@ -805,25 +973,61 @@ __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
     }
   };
 
+  // A partial item (equal ranges): the normalised fp32 O of each 16-row block
+  // and 16-dim block as the lanes hold it (1 KiB per store), and the rows'
+  // log2-sum-exp.  More operations than store_out's SOPS, which the waits
+  // count: they are then stricter than they need be.
+  [[maybe_unused]] float m_part[QS];
+  auto store_part = [&](const Item &it) {
+    const float vscale = FP8 ? ld_const(a.v_scale + it.kvh) : 1.f;
+#pragma unroll
+    for (int qs = 0; qs < QS; ++qs) {
+      const float l = sum32(sum16(lsum[qs]));
+      const float inv = (l > 0.f ? 1.0f / l : 0.f) * vscale;
+      const int64_t unit = (static_cast<int64_t>(it.part) * NW + wave) * QS + qs;
+      f32x4 *po = reinterpret_cast<f32x4 *>(a.part_o) + unit * DT::NJ * 64 + lane;
+#pragma unroll
+      for (int j = 0; j < DT::NJ; ++j) po[j * 64] = o[qs][j] * inv;
+      if (g == 0) a.part_l[unit * 16 + m] = l > 0.f ? m_part[qs] + __log2f(l) : kNegInf;
+    }
+  };
   auto store_out = [&](const Item &it) {
+    if (RANGES && it.part >= 0) {
+      store_part(it);
+      return;
+    }
     if constexpr (GATED) store_out_gated(it);
     else store_out_plain(it);
   };
 
   // ----------------------------------------------------------------- queue
-  if (threadIdx.x == 0) {
+  if (!RANGES && threadIdx.x == 0) {
     lds_item[0] = static_cast<int>(atomicAdd(ctr, 1u));
     lds_item[1] = static_cast<int>(atomicAdd(ctr, 1u));
   }
   __syncthreads();
-  const int n_items = a.by_cost ? __builtin_amdgcn_readfirstlane(*lds_n) : cx * n_x;
+  // Equal ranges: the next piece, its descriptor written for the merge.
+  [[maybe_unused]] auto take = [&]() {
+    const Item it = range_next(a, cq, rg, paged ? a.block_size / kKeys : 1);
+    if (it.live && it.part >= 0 && threadIdx.x == 0)
+      a.part_desc[it.part] = int4{it.s, it.head0, it.row_begin, it.last ? kPieceLast : kPieceMore};
+    return it;
+  };
+  const int n_items = RANGES ? 1 : a.by_cost ? __builtin_amdgcn_readfirstlane(*lds_n) : cx * n_x;
   auto describe = [&](int idx) {
     if constexpr (TAB) return describe_by_table(a, cq, idx, n_items);
     else return a.by_cost ? describe_by_cost(a, cq, idx, n_items) : describe_by_tile<S>(a, idx, n_items, n_x, n_y, cx, x);
   };
-  int idx_cur = __builtin_amdgcn_readfirstlane(lds_item[0]);
-  int idx_nxt = __builtin_amdgcn_readfirstlane(lds_item[1]);
-  Item cur = describe(idx_cur);
+  // (equal ranges: 0 for a piece, 1 past the range's end)
+  int idx_cur = RANGES ? 0 : __builtin_amdgcn_readfirstlane(lds_item[0]);
+  int idx_nxt = RANGES ? 0 : __builtin_amdgcn_readfirstlane(lds_item[1]);
+  Item cur;
+  if constexpr (RANGES) {
+    cur = take();
+    idx_cur = cur.live ? 0 : 1;
+  } else {
+    cur = describe(idx_cur);
+  }
   // The next item: described one ahead and kept, or -- from the list, where
   // describing is cheap -- described again where it is used, so its fields
   // hold no registers through the tile loops.  Measured with the list:
@@ -831,7 +1035,12 @@ __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
   // 96 fewer scalar spills), keeping the item at 256 (-3%).
   constexpr bool kRedescribe = TAB && D == 128;
   Item nxt{};
-  if constexpr (!kRedescribe) nxt = describe(idx_nxt);
+  if constexpr (RANGES) {
+    nxt = take();
+    idx_nxt = nxt.live ? 0 : 1;
+  } else if constexpr (!kRedescribe) {
+    nxt = describe(idx_nxt);
+  }
   auto next_item = [&]() -> Item {
     if constexpr (kRedescribe) return describe(idx_nxt);
     else return nxt;
@@ -855,7 +1064,7 @@ __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
     // compiler's own wait for the result (at the end of the item) count
     // them; the copies in flight then need not complete.
     uint32_t fetched;
-    if (threadIdx.x == 0) fetched = atomicAdd(ctr, 1u);
+    if (!RANGES && threadIdx.x == 0) fetched = atomicAdd(ctr, 1u);
     load_q(cur);
     asm volatile("" ::: "memory");  // the padding stays behind the Q loads
     {
@@ -890,7 +1099,7 @@ __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
       const int wave_key_end = a.causal ? min(Lk, wrow_last + P + 1) : Lk;
       // Tiles this wave computes (a prefix: a causal wave stops at its own
       // diagonal) and, among them, the leading tiles that need no mask.
-      const int wave_nkt = wave_live ? min(n_kt, (wave_key_end + kKeys - 1) / kKeys) : 0;
+      const int wave_nkt = wave_live ? max(0, min(n_kt, (wave_key_end + kKeys - 1) / kKeys)) : 0;
       int n_plain = min(wave_nkt, Lk / kKeys);
       if (a.causal) n_plain = min(n_plain, max(0, wrow0 + P + 1) / kKeys);
       const int32_t *bt_row = paged ? a.block_tables + static_cast<int64_t>(cur.s) * a.bt_stride : nullptr;
@@ -1186,7 +1395,7 @@ __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
       // Whether the block of key tile jt exists (the masked loop once a
       // missing block has been seen).
       auto block_ok = [&](int jt) {
-        const int blk = ld_const(bt_row + jt * kKeys / a.block_size);
+        const int blk = ld_const(bt_row + (RANGES ? cur.blk0 : 0) + jt * kKeys / a.block_size);
         return blk >= 0 && blk < num_blocks;
       };
 
@@ -1238,6 +1447,10 @@ __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
         if (pend) rescale(alpha);
         pv_only(vf, pb);
       }
+      if constexpr (RANGES) {
+#pragma unroll
+        for (int qs = 0; qs < QS; ++qs) m_part[qs] = m_use[qs];
+      }
     } else {
       queue_copy(next_item());
     }
@@ -1245,6 +1458,15 @@ __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
     // reading slot k + 1 cannot be overtaken, the write comes after the
     // barrier that follows its read).  A plain barrier: the fence of
     // __syncthreads() would wait for the K/V copies in flight.
+    if constexpr (RANGES) {
+      raw_barrier();
+      prev = cur;
+      cur = nxt;
+      idx_cur = idx_nxt;
+      nxt = take();
+      idx_nxt = nxt.live ? 0 : 1;
+      continue;
+    }
     if (threadIdx.x == 0) {
       lds_item[(k + 2) & 3] = static_cast<int>(fetched);
       wait_lgkmcnt0();
@@ -1262,7 +1484,7 @@ __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
     idx_nxt = idx_new;
   }
   wait_vmcnt<0>();  // the stream's last (empty) copies and the last stores complete before the workgroup ends
-  if (threadIdx.x == 0) {
+  if (!RANGES && threadIdx.x == 0) {
     if (atomicAdd(a.queue + 8, 1u) == gridDim.x - 1) {
       // Every other workgroup has taken its last index and finished.
 #pragma unroll
@@ -1273,14 +1495,148 @@ __device__ __forceinline__ void prefill_persistent(const PrefillArgs &a) {
 
 // The body lives in a device function: its inline assembly uses register
 // constraints that only the device compilation accepts.
-template <class T, int D, class S, bool GATED, bool FP8, bool TAB>
+template <class T, int D, class S, bool GATED, bool FP8, int MODE>
 __global__ __launch_bounds__(64 * S::NW) __attribute__((amdgpu_waves_per_eu(S::WPE)))
 void varlen_prefill_dma_kernel(const PrefillArgs a) {
-  prefill_persistent<T, D, S, GATED, FP8, TAB>(a);
+  prefill_persistent<T, D, S, GATED, FP8, MODE>(a);
 }
 
+// Merge of the items cut by equal ranges: workgroups lin handle the item
+// whose first piece lies in slot 2 lin + 1; its later pieces are the slots 2j
+// of the ranges after it (of the same queue, n_wg ranges each) up to the one
+// marked last.  One wave per 16 rows of one head (the unit a wave of the main
+// kernel wrote) and kMergeJ of its 16-dim blocks.  Latency-bound and
+// bandwidth-bound alike (a few hundred items of 2-4 pieces of 64 KiB): the
+// descriptors of 64 ranges are read at once, then everything of up to 4
+// pieces, so an item takes two round trips to memory before its store.  A
+// launch's merge takes 12-16 us; loading the pieces one after another, with
+// whole rows per wave, 12-17.
+constexpr int kMergeJ = 4;
+template <class T, int D, class S>
+__global__ __launch_bounds__(64 * S::NW * S::QS) void prefill_merge_kernel(const PrefillArgs a, int n_wg) {
+  using DT = DTile<T, D>;
+  constexpr int kUnits = S::NW * S::QS, kChunk = 4;
+  const int lin = blockIdx.x;
+  const int lane = threadIdx.x & 63, unit = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m = lane & 15, g = lane >> 4;
+  const int q_end = (lin / n_wg + 1) * n_wg;  // past the queue's last range
+  auto later = [&](int base) { return base + lane < q_end ? a.part_desc[2 * (base + lane)].w : kPieceNone; };
+  const int4 d = a.part_desc[2 * lin + 1];
+  int base = lin + 1;
+  int w = later(base);
+  if (d.w == kPieceNone) return;
+  const int wave = unit / S::QS, qs = unit % S::QS;
+  const int q0 = ld_const(a.cu_q + d.x), Lq = ld_const(a.cu_q + d.x + 1) - q0;
+  float M = kNegInf, W = 0.f;
+  f32x4 acc[kMergeJ];
+#pragma unroll
+  for (int j = 0; j < kMergeJ; ++j) acc[j] = f32x4{0, 0, 0, 0};
+  bool more = true;
+  uint64_t has = 0;  // the pieces of ranges base + bit not yet taken
+  auto scan = [&]() {
+    has = __builtin_amdgcn_ballot_w64(w != kPieceNone);
+    const uint64_t fin = __builtin_amdgcn_ballot_w64(w == kPieceLast);
+    if (fin != 0) {
+      has &= (fin & -fin) | ((fin & -fin) - 1);  // up to the item's last piece
+      more = false;
+    }
+  };
+  scan();
+  int slot = 2 * lin + 1;  // the next piece (-1: none)
+  while (slot >= 0) {
+    int sl[kChunk];
+#pragma unroll
+    for (int i = 0; i < kChunk; ++i) {
+      sl[i] = slot;
+      slot = -1;
+      while (has == 0 && more && base + 64 < q_end) {  // the next 64 ranges
+        base += 64;
+        w = later(base);
+        scan();
+      }
+      if (has != 0) {
+        slot = 2 * (base + static_cast<int>(__builtin_ctzll(has)));
+        has &= has - 1;
+      }
+    }
+    float l[kChunk];
+    f32x4 p[kChunk][kMergeJ];
+#pragma unroll
+    for (int i = 0; i < kChunk; ++i) {
+      l[i] = kNegInf;
+      if (sl[i] >= 0) {
+        const int64_t u = static_cast<int64_t>(sl[i]) * kUnits + unit;
+        l[i] = a.part_l[u * 16 + m];
+        const f32x4 *po = reinterpret_cast<const f32x4 *>(a.part_o) + (u * DT::NJ + kMergeJ * blockIdx.y) * 64 + lane;
+#pragma unroll
+        for (int j = 0; j < kMergeJ; ++j) p[i][j] = po[j * 64];
+      }
+    }
+    float mc = M;
+#pragma unroll
+    for (int i = 0; i < kChunk; ++i) mc = fmaxf(mc, l[i]);
+    if (mc == kNegInf) mc = 0.f;  // no piece has a visible key yet: weights 0
+    const float f = __builtin_amdgcn_exp2f(M - mc);
+    W *= f;
+#pragma unroll
+    for (int j = 0; j < kMergeJ; ++j) acc[j] *= f;
+#pragma unroll
+    for (int i = 0; i < kChunk; ++i)
+      if (sl[i] >= 0) {
+        const float wt = __builtin_amdgcn_exp2f(l[i] - mc);
+        W += wt;
+#pragma unroll
+        for (int j = 0; j < kMergeJ; ++j) acc[j] += p[i][j] * wt;
+      }
+    M = mc;
+  }
+  const float inv = W > 0.f ? 1.0f / W : 0.f;
+  const int row = d.z + 16 * S::QS * (wave / a.G4) + 16 * qs + m;
+  if (row >= Lq) return;
+  const int64_t head = d.y + wave % a.G4;
+  const int64_t dim = 2 * (16 * kMergeJ * static_cast<int>(blockIdx.y) + 4 * g);
+  uint8_t *op = a.out + (q0 + row) * a.o_rs + head * a.o_hs + dim;
+  const uint8_t *gp = a.gate ? a.gate + (q0 + row) * a.g_rs + head * a.g_hs + dim : nullptr;
+#pragma unroll
+  for (int j = 0; j < kMergeJ; ++j) {
+    const f32x4 v = acc[j] * inv;
+    *reinterpret_cast<u32x2 *>(op + 32 * j) =
+        gp ? gate4<T>(v, *reinterpret_cast<const u32x2 *>(gp + 32 * j)) : u32x2{T::pack2(v[0], v[1]), T::pack2(v[2], v[3])};
+  }
+}
+
+// Whether a launch runs as equal ranges, and the bytes of its partial
+// outputs: two slots per resident workgroup.  The items (rows of each
+// sequence in tiles, per kv-head slot) are bounded from the sizes the host
+// knows.  Up to kRangeWaves items per resident workgroup: a single causal
+// prompt with more has no item longer than a workgroup's share.  Beyond, the
+// dynamic queue balances by itself: 16 prompts with 7.4 items per workgroup
+// 289 us whole, 323 as ranges; 6 at head_dim 256 with 5.2 items 303 and 391; at
+// 3.9 items (4 kv heads) 178 and 175.
+template <int D, class S>
+struct RangePlan {
+  static constexpr int64_t kSlotO = static_cast<int64_t>(S::NW) * S::QS * (D / 16) * 1024;
+  static constexpr int64_t kSlotL = static_cast<int64_t>(S::NW) * S::QS * 64;
+  static int grid() { return (device_cus() * S::WG_PER_CU + 7) / 8 * 8; }
+  static int64_t bytes() { return 2 * grid() * (kSlotO + kSlotL + static_cast<int64_t>(sizeof(int4))); }
+  // Entries of a queue's list (an upper bound on what the kernel forms).
+  static int64_t entries(int num_seqs, int n_qtiles, int n_y) {
+    const int rl = shared_slots_log2(n_y);
+    const int64_t U = static_cast<int64_t>(n_y) * num_seqs;
+    const int64_t w = rl > 0 ? 1 : (U >= 8 ? (n_y + 7) / 8 : n_y);
+    return num_seqs * static_cast<int64_t>((n_qtiles + (1 << rl) - 1) >> rl) * w;
+  }
+  static bool use(int num_seqs, int64_t total_q, int max_seqlen_q, int max_seqlen_k, int n_y, int G4) {
+    const int rows = S::ITEM_ROWS / G4;
+    const int n_qtiles = (max_seqlen_q + rows - 1) / rows;
+    const int64_t items = std::min<int64_t>((total_q + rows - 1) / rows + num_seqs, static_cast<int64_t>(num_seqs) * n_qtiles) * n_y;
+    return num_seqs <= kMaxSeqs && entries(num_seqs, n_qtiles, n_y) < S::MAX_ITEMS &&
+           max_seqlen_k >= kRangeKeys && items < kRangeWaves * grid();
+  }
+};
+
 template <class T, int D, class S, bool FP8>
-int launch_prefill_dma(PrefillArgs a, hipStream_t st) {
+int launch_prefill_dma(PrefillArgs a, int64_t total_q, uint8_t *split_ws, int64_t split_bytes, hipStream_t st) {
   const int rows_per_item = S::ITEM_ROWS / a.G4;
   a.n_qtiles = (a.max_seqlen_q + rows_per_item - 1) / rows_per_item;
   const int64_t U = static_cast<int64_t>(a.Hkv) * a.quads * a.num_seqs;
@@ -1288,6 +1644,23 @@ int launch_prefill_dma(PrefillArgs a, hipStream_t st) {
   if (total > 0x7fffffff) return fail(NQ_EINVAL, "varlen_prefill: too many work items");
   if (!a.queue) return fail(NQ_EINVAL, "varlen_prefill: null workspace");
   a.pin = U >= 8;
+  using RP = RangePlan<D, S>;
+  if (split_ws && split_bytes >= RP::bytes() &&
+      RP::use(a.num_seqs, total_q, a.max_seqlen_q, a.max_seqlen_k, a.Hkv * a.quads, a.G4)) {
+    const int grid = RP::grid();
+    a.rep_log2 = shared_slots_log2(a.Hkv * a.quads);
+    if (a.rep_log2 > 0) a.pin = 1;
+    a.part_o = reinterpret_cast<float *>(split_ws);
+    a.part_l = reinterpret_cast<float *>(split_ws + 2 * grid * RP::kSlotO);
+    a.part_desc = reinterpret_cast<int4 *>(split_ws + 2 * grid * (RP::kSlotO + RP::kSlotL));
+    auto *kern = a.gate ? varlen_prefill_dma_kernel<T, D, S, true, FP8, 2> : varlen_prefill_dma_kernel<T, D, S, false, FP8, 2>;
+    kern<<<grid, 64 * S::NW, S::LDS_BYTES, st>>>(a);
+    const int rc = check_launch("varlen_prefill(ranges)");
+    if (rc != NQ_OK) return rc;
+    prefill_merge_kernel<T, D, S>
+        <<<dim3(grid, D / 16 / kMergeJ), 64 * S::NW * S::QS, 0, st>>>(a, a.pin ? grid / 8 : grid);
+    return check_launch("varlen_prefill(merge)");
+  }
   // Cost order when the sequence bounds fit in LDS and counting the items
   // at launch stays short; query-tile order otherwise.
   a.by_cost = a.num_seqs <= kMaxSeqs && static_cast<int64_t>(a.num_seqs) * a.n_qtiles <= 65536;
@@ -1299,17 +1672,8 @@ int launch_prefill_dma(PrefillArgs a, hipStream_t st) {
   // (its groups x query tiles bound it), the (level, sequence) starts fit the
   // ring and the packed words hold the fields.
   const int64_t cx_max = U >= 8 ? (U + 7) / 8 : U;
-  // Fewer than 8 kv-head slots that divide 8: each slot belongs to 8 / n_y
-  // XCDs, which take its query tiles in turn, so that every XCD carries the
-  // same work whatever the lengths (with groups pinned whole, 4 slots put the
-  // even sequences on one half of the XCDs and the odd ones on the other:
-  // 6 prompts of 333-2567 tokens, 4 kv heads of 256, 349 -> 255 us; 16 prompts
-  // of 256-2048 behind prefixes, 4 kv heads of 128, 215 -> 178 us).  A slot's
-  // K/V is then read into 2, 4 or 8 L2s instead of one.
-  const int n_y = a.Hkv * a.quads;
-  int rep_log2 = 0;
-  while (n_y << rep_log2 < 8) ++rep_log2;
-  if (n_y << rep_log2 == 8 && rep_log2 > 0 &&
+  const int rep_log2 = shared_slots_log2(a.Hkv * a.quads);
+  if (rep_log2 > 0 &&
       static_cast<int64_t>(a.num_seqs) * ((a.n_qtiles + (1 << rep_log2) - 1) >> rep_log2) <= S::MAX_ITEMS)
     a.rep_log2 = rep_log2;
   if (a.by_cost && (a.rep_log2 > 0 || cx_max * a.n_qtiles <= S::MAX_ITEMS) && static_cast<int64_t>(a.num_seqs) * a.n_levels * 4 <= S::RING_BYTES &&
@@ -1324,20 +1688,20 @@ int launch_prefill_dma(PrefillArgs a, hipStream_t st) {
   // items; a multiple of 8 so every XCD gets the same count.
   int64_t grid = (static_cast<int64_t>(device_cus()) * S::WG_PER_CU + 7) / 8 * 8;
   if (grid > total) grid = total;  // work_grid() is a multiple of 8 when pinned
-  auto *kern = a.gate ? (a.by_cost == 2 ? varlen_prefill_dma_kernel<T, D, S, true, FP8, true>
-                                        : varlen_prefill_dma_kernel<T, D, S, true, FP8, false>)
-                     : (a.by_cost == 2 ? varlen_prefill_dma_kernel<T, D, S, false, FP8, true>
-                                        : varlen_prefill_dma_kernel<T, D, S, false, FP8, false>);
+  auto *kern = a.gate ? (a.by_cost == 2 ? varlen_prefill_dma_kernel<T, D, S, true, FP8, 1>
+                                        : varlen_prefill_dma_kernel<T, D, S, true, FP8, 0>)
+                     : (a.by_cost == 2 ? varlen_prefill_dma_kernel<T, D, S, false, FP8, 1>
+                                        : varlen_prefill_dma_kernel<T, D, S, false, FP8, 0>);
   kern<<<static_cast<int>(grid), 64 * S::NW, S::LDS_BYTES, st>>>(a);
   return check_launch(a.gate ? "varlen_prefill(gated)" : "varlen_prefill");
 }
 
 template <class T, bool FP8, int D>
-int launch_prefill(PrefillArgs a, hipStream_t s) {
+int launch_prefill(const PrefillArgs &a, int64_t total_q, uint8_t *split_ws, int64_t split_bytes, hipStream_t s) {
   if constexpr (D == 256) {
-    return launch_prefill_dma<T, D, ShapeD, FP8>(a, s);
+    return launch_prefill_dma<T, D, ShapeD, FP8>(a, total_q, split_ws, split_bytes, s);
   } else {
-    return launch_prefill_dma<T, D, ShapeC, FP8>(a, s);  // fp8 copies: one 1 KiB piece per wave
+    return launch_prefill_dma<T, D, ShapeC, FP8>(a, total_q, split_ws, split_bytes, s);  // fp8 copies: one 1 KiB piece per wave
   }
 }
 
@@ -1357,7 +1721,7 @@ static int varlen_prefill_impl(const void *q, int64_t q_row_stride, int64_t q_he
                                float softmax_scale, int causal, int q_dtype, int kv_dtype, const float *k_scale,
                                const float *v_scale, void *workspace, int64_t workspace_bytes, const void *gate,
                                int64_t gate_row_stride, int64_t gate_head_stride, int64_t total_q,
-                               void *stream) {
+                               void *split_workspace, int64_t split_bytes, void *stream) {
   if (num_seqs == 0 || max_seqlen_q == 0) return NQ_OK;
   if (num_seqs < 0 || max_seqlen_q < 0 || max_seqlen_k < 0 || num_q_heads <= 0 || num_kv_heads <= 0)
     return fail(NQ_EINVAL, "varlen_prefill: bad sizes");
@@ -1438,16 +1802,19 @@ static int varlen_prefill_impl(const void *q, int64_t q_row_stride, int64_t q_he
   a.k_scale = k_scale;
   a.v_scale = v_scale;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  uint8_t *sw = static_cast<uint8_t *>(split_workspace);
+  if (sw && (!aligned(sw, 256) || total_q < 0))
+    return fail(NQ_EINVAL, "varlen_prefill: split workspace alignment or total_q");
   int rc;
   if (head_dim == 256) {
     if (q_dtype == NQ_BF16)
-      rc = fp8 ? launch_prefill<BF16, true, 256>(a, st) : launch_prefill<BF16, false, 256>(a, st);
+      rc = fp8 ? launch_prefill<BF16, true, 256>(a, total_q, sw, split_bytes, st) : launch_prefill<BF16, false, 256>(a, total_q, sw, split_bytes, st);
     else
-      rc = fp8 ? launch_prefill<F16, true, 256>(a, st) : launch_prefill<F16, false, 256>(a, st);
+      rc = fp8 ? launch_prefill<F16, true, 256>(a, total_q, sw, split_bytes, st) : launch_prefill<F16, false, 256>(a, total_q, sw, split_bytes, st);
   } else if (q_dtype == NQ_BF16) {
-    rc = fp8 ? launch_prefill<BF16, true, 128>(a, st) : launch_prefill<BF16, false, 128>(a, st);
+    rc = fp8 ? launch_prefill<BF16, true, 128>(a, total_q, sw, split_bytes, st) : launch_prefill<BF16, false, 128>(a, total_q, sw, split_bytes, st);
   } else {
-    rc = fp8 ? launch_prefill<F16, true, 128>(a, st) : launch_prefill<F16, false, 128>(a, st);
+    rc = fp8 ? launch_prefill<F16, true, 128>(a, total_q, sw, split_bytes, st) : launch_prefill<F16, false, 128>(a, total_q, sw, split_bytes, st);
   }
   return rc;
 }
@@ -1465,7 +1832,7 @@ extern "C" int nq_varlen_prefill(const void *q, int64_t q_row_stride, int64_t q_
                              max_seqlen_q, max_seqlen_k, block_tables, bt_stride, max_blocks_per_seq, num_blocks,
                              out, out_row_stride, out_head_stride, num_seqs, num_q_heads, num_kv_heads, head_dim,
                              block_size, softmax_scale, causal, q_dtype, kv_dtype, k_scale, v_scale, workspace,
-                             workspace_bytes, nullptr, 0, 0, 0, stream);
+                             workspace_bytes, nullptr, 0, 0, 0, nullptr, 0, stream);
 }
 
 extern "C" int nq_varlen_prefill_gated(
@@ -1481,5 +1848,37 @@ extern "C" int nq_varlen_prefill_gated(
                              max_seqlen_q, max_seqlen_k, block_tables, bt_stride, max_blocks_per_seq, num_blocks,
                              out, out_row_stride, out_head_stride, num_seqs, num_q_heads, num_kv_heads, head_dim,
                              block_size, softmax_scale, causal, q_dtype, kv_dtype, k_scale, v_scale, workspace,
-                             workspace_bytes, gate, gate_row_stride, gate_head_stride, total_q, stream);
+                             workspace_bytes, gate, gate_row_stride, gate_head_stride, total_q, nullptr, 0, stream);
+}
+
+extern "C" int64_t nq_prefill_split_workspace_bytes(int num_seqs, int64_t total_q, int max_seqlen_q, int max_seqlen_k,
+                                                    int num_q_heads, int num_kv_heads, int head_dim) {
+  if (num_seqs <= 0 || total_q <= 0 || max_seqlen_q <= 0 || max_seqlen_k <= 0 || num_kv_heads <= 0 ||
+      num_q_heads < num_kv_heads || num_q_heads % num_kv_heads != 0)
+    return 0;
+  const int G = num_q_heads / num_kv_heads, G4 = G < 4 ? G : 4, n_y = num_kv_heads * (G < 4 ? 1 : G / 4);
+  if ((G > 4 && G % 4 != 0) || G == 3) return 0;
+  if (head_dim == 128)
+    return RangePlan<128, ShapeC>::use(num_seqs, total_q, max_seqlen_q, max_seqlen_k, n_y, G4)
+               ? RangePlan<128, ShapeC>::bytes() : 0;
+  if (head_dim == 256)
+    return RangePlan<256, ShapeD>::use(num_seqs, total_q, max_seqlen_q, max_seqlen_k, n_y, G4)
+               ? RangePlan<256, ShapeD>::bytes() : 0;
+  return 0;
+}
+
+extern "C" int nq_varlen_prefill_split(
+    const void *q, int64_t q_row_stride, int64_t q_head_stride, const void *k, const void *v,
+    int64_t kv_row_stride, const int32_t *cu_seqlens_q, const int32_t *cu_seqlens_k, int max_seqlen_q,
+    int max_seqlen_k, const int32_t *block_tables, int64_t bt_stride, int max_blocks_per_seq, int64_t num_blocks,
+    void *out, int64_t out_row_stride, int64_t out_head_stride, int num_seqs, int num_q_heads, int num_kv_heads,
+    int head_dim, int block_size, float softmax_scale, int causal, int q_dtype, int kv_dtype, const float *k_scale,
+    const float *v_scale, void *workspace, int64_t workspace_bytes, const void *gate, int64_t gate_row_stride,
+    int64_t gate_head_stride, int64_t total_q, void *split_workspace, int64_t split_workspace_bytes, void *stream) {
+  return varlen_prefill_impl(q, q_row_stride, q_head_stride, k, v, kv_row_stride, cu_seqlens_q, cu_seqlens_k,
+                             max_seqlen_q, max_seqlen_k, block_tables, bt_stride, max_blocks_per_seq, num_blocks,
+                             out, out_row_stride, out_head_stride, num_seqs, num_q_heads, num_kv_heads, head_dim,
+                             block_size, softmax_scale, causal, q_dtype, kv_dtype, k_scale, v_scale, workspace,
+                             workspace_bytes, gate, gate_row_stride, gate_head_stride, total_q, split_workspace,
+                             split_workspace_bytes, stream);
 }

@@ -31,6 +31,7 @@ from ._lib import check, dtype_code, lib, ptr, require_cuda, stream_of
 # buffer once no captured graph that used them will be replayed.
 _workspaces: dict[tuple[int, int], torch.Tensor] = {}
 _prefill_queues: dict[tuple[int, int], torch.Tensor] = {}
+_prefill_parts: dict[tuple[int, int], torch.Tensor] = {}
 _retired: list[torch.Tensor] = []
 _DEBUG_QUEUE = os.environ.get("NQ_DEBUG_PREFILL_QUEUE", "0") not in ("", "0")
 
@@ -60,14 +61,14 @@ def _grow(table, key, nbytes, dtype, device, zero=False):
 
 def release_workspaces(device=None) -> int:
     """Drop the kernels' per-stream buffers (decode split-K workspaces,
-    prefill queue counters) and every retired buffer, of ``device`` or of
+    prefill queue counters and partial outputs) and every retired buffer, of ``device`` or of
     all devices; returns how many were dropped.  Only safe once no HIP graph
     captured with them will be replayed again: a replay would write freed
     memory.  Later calls allocate fresh buffers (the prefill counters start
     at zero again)."""
     idx = None if device is None else _key(device)[0]
     n = 0
-    for table in (_workspaces, _prefill_queues):
+    for table in (_workspaces, _prefill_queues, _prefill_parts):
         for key in [k for k in table if idx is None or k[0] == idx]:
             del table[key]
             n += 1
@@ -308,14 +309,21 @@ def varlen_prefill(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen
             out.stride(0), out.stride(1), n, hq, hkv, d, bs, float(softmax_scale), 1 if causal else 0,
             dtype_code(q.dtype), dtype_code(k.dtype), ptr(k_scale) if fp8 else None,
             ptr(v_scale) if fp8 else None, ptr(ws), ws.numel() * 4)
-    if gate is None:
-        rc = lib().nq_varlen_prefill(*args, stream_of(q))
-    else:
+    g3 = None
+    if gate is not None:
         require_cuda(gate, what="varlen_prefill")
         if gate.dtype != q.dtype:
             raise RuntimeError("varlen_prefill: gate dtype must match q")
         g3 = _gate3(gate, tq, hq, d, "varlen_prefill")
-        rc = lib().nq_varlen_prefill_gated(*args, ptr(g3), g3.stride(0), g3.stride(1), tq, stream_of(q))
+    gargs = (None, 0, 0) if g3 is None else (ptr(g3), g3.stride(0), g3.stride(1))
+    part_bytes = lib().nq_prefill_split_workspace_bytes(n, tq, int(max_seqlen_q), int(max_seqlen_k), hq, hkv, d)
+    if part_bytes > 0:    # too few work items for the chip: equal key ranges, then a merge
+        parts = _grow(_prefill_parts, _key(q.device), part_bytes, torch.uint8, q.device)
+        rc = lib().nq_varlen_prefill_split(*args, *gargs, tq, ptr(parts), parts.numel(), stream_of(q))
+    elif g3 is None:
+        rc = lib().nq_varlen_prefill(*args, stream_of(q))
+    else:
+        rc = lib().nq_varlen_prefill_gated(*args, *gargs, tq, stream_of(q))
     check(rc, "varlen_prefill")
     if _DEBUG_QUEUE:
         _check_queue_zero(ws)

@@ -1,4 +1,5 @@
-"""Prefill work distribution on the GPU: kv-head slots shared by several XCDs.
+"""Prefill work distribution on the GPU: kv-head slots shared by several XCDs,
+and launches cut into equal key ranges whose partial outputs are merged.
 
 Every output row against the float32 device reference (oracle/sdpa_path), a
 few rows against the float64 oracle.
@@ -6,9 +7,11 @@ few rows against the float64 oracle.
 import pytest
 import torch
 
+from nano_qwen_amd import kernels
+from nano_qwen_amd._lib import lib
 from oracle.inputs import make_prefill_case
 from tests.parity import TOL_BF16, TOL_FP8
-from tests.test_gpu_prefill import check
+from tests.test_gpu_prefill import check, run_step
 
 pytestmark = pytest.mark.gpu
 
@@ -23,3 +26,46 @@ def test_prefill_shared_slots(cuda, hq, hkv, d):
         case = make_prefill_case("cfg3", seed=hq + hkv, device=cuda, nseq=7, lq=(1, 700), prefix_blocks=prefix, hq=hq,
                                  hkv=hkv, d=d)
         check(case, range(7), TOL_BF16, rows_per_seq=6, all_rows=True)
+
+
+def _ranges(case):
+    return lib().nq_prefill_split_workspace_bytes(case["nseq"], case["q"].shape[0], case["max_seqlen_q"],
+                                                  case["max_seqlen_k"], case["hq"], case["hkv"], case["d"]) > 0
+
+
+@pytest.mark.parametrize("kw", [
+    dict(nseq=1, lq=(1111, 1111), prefix_blocks=(0, 0)),                 # packed, cuts at any tile
+    dict(nseq=3, lq=(1, 900), prefix_blocks=(0, 0), hq=8, hkv=2),        # packed, shared slots
+    dict(nseq=1, lq=(1, 1), prefix_blocks=(31, 31)),                     # one row, one item per kv head
+    dict(nseq=4, lq=(20, 300), prefix_blocks=(9, 20)),                   # paged, half without a prefix
+    dict(nseq=4, lq=(20, 300), prefix_blocks=(9, 20), dtype=torch.float16, hq=64),
+    dict(nseq=3, lq=(33, 200), prefix_blocks=(7, 24), kv="fp8"),
+    dict(nseq=2, lq=(64, 700), prefix_blocks=(0, 6), hq=16, hkv=4, d=256),
+    dict(nseq=2, lq=(64, 300), prefix_blocks=(4, 9), hq=16, hkv=2, d=256, kv="fp8"),
+    dict(nseq=2, lq=(64, 500), prefix_blocks=(2, 3), hq=12, hkv=3),      # slots that do not divide 8
+], ids=str)
+def test_prefill_ranges(cuda, kw):
+    tol = TOL_FP8 if kw.get("kv") == "fp8" else TOL_BF16
+    case = make_prefill_case("cfg3", seed=3, device=cuda, **kw)
+    assert _ranges(case)
+    check(case, range(kw["nseq"]), tol, rows_per_seq=8, all_rows=True)
+
+
+def test_prefill_ranges_gate_and_reuse(cuda):
+    """Gated = the eager gate of the ungated output (at most one ulp on 0.1% of
+    elements, as for whole items); a smaller launch that reuses the partial
+    buffer of a larger one does not see its pieces; a repeat is bit-identical."""
+    big = make_prefill_case("cfg3", seed=5, device=cuda, nseq=4, lq=(100, 300), prefix_blocks=(9, 20))
+    small = make_prefill_case("cfg3", seed=6, device=cuda, nseq=1, lq=(90, 90), prefix_blocks=(3, 3))
+    assert _ranges(big) and _ranges(small)
+    first = run_step(small)
+    out = run_step(big)
+    assert torch.equal(run_step(small), first)
+    assert torch.equal(run_step(big), out)
+    gate = torch.randn(out.shape, generator=torch.Generator(device=cuda).manual_seed(1), device=cuda).to(out.dtype)
+    got = kernels.varlen_prefill(big["q"], big["k_cache"], big["v_cache"], big["cu_seqlens_q"], big["cu_seqlens_k"],
+                                 big["max_seqlen_q"], big["max_seqlen_k"], big["scale"],
+                                 block_table=big["block_tables"], gate=gate)
+    want = out * torch.sigmoid(gate)
+    off = (got.view(torch.int16).int() - want.view(torch.int16).int()).abs()
+    assert int(off.max()) <= 1 and float((off > 0).float().mean()) <= 1e-3
