@@ -469,6 +469,31 @@ int nq_gdn_prefill(const void *q, int64_t q_row_stride, const void *k, int64_t k
                    int head_k_dim, int head_v_dim, int dtype, void *stream);
 
 /*
+ * nq_gdn_prefill with room for segment states, for launches with few
+ * sequences: their chunks form chains that leave most of the device idle, so
+ * each sequence is cut into segments that run side by side, once for their
+ * states and once, after a float32 chaining of those, for the outputs (same
+ * results up to the order of float32 sums).  total_tokens: rows of q.  A null
+ * or smaller workspace than nq_gdn_prefill_workspace_bytes, or a launch for
+ * which that is 0, runs as nq_gdn_prefill.  workspace must be 256-byte
+ * aligned; its contents need no clearing.  Calls that overlap may not share
+ * one.
+ */
+int nq_gdn_prefill_split(const void *q, int64_t q_row_stride, const void *k, int64_t k_row_stride,
+                         const void *v, int64_t v_row_stride, const void *a, int64_t a_row_stride,
+                         const void *b, int64_t b_row_stride, const float *A_log, const float *dt_bias,
+                         const int32_t *cu_seqlens, int num_seqs, float *state,
+                         const int32_t *state_indices, int64_t num_slots, int initial_state_from_slot,
+                         void *out, int64_t out_row_stride, int num_k_heads, int num_v_heads,
+                         int head_k_dim, int head_v_dim, int dtype, int64_t total_tokens,
+                         void *workspace, int64_t workspace_bytes, void *stream);
+
+/* Bytes of workspace with which nq_gdn_prefill_split cuts a launch of these
+ * sizes into segments; 0: it would not (decided from the sizes and the current
+ * device alone). */
+int64_t nq_gdn_prefill_workspace_bytes(int num_seqs, int64_t total_tokens, int num_v_heads);
+
+/*
  * Gated RMS norm of the Gated DeltaNet output, one pass.
  * Replaces RMSNormGated.forward (layers/layernorm.py:143-157) as applied by
  * GatedDeltaNet (self.norm(out, z), layers/gated_delta_net.py:205-207,

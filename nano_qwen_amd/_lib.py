@@ -76,6 +76,11 @@ _SIGS = {
     "nq_gdn_prefill": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64,
                                c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                                c_int64, c_int, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int, c_void_p]),
+    "nq_gdn_prefill_split": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64,
+                                     c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
+                                     c_int64, c_int, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int, c_int64,
+                                     c_void_p, c_int64, c_void_p]),
+    "nq_gdn_prefill_workspace_bytes": (c_int64, [c_int, c_int64, c_int]),
     "nq_gated_rmsnorm": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_float, c_void_p, c_int64,
                                  c_int64, c_int, c_int, c_void_p]),
     "nq_gdn_conv1d": (c_int, [c_void_p, c_int64, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_int64,

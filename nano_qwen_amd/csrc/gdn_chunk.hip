@@ -48,6 +48,24 @@
 // LDS tiles are row-major with 16-byte chunks XOR-swizzled per row (128-
 // column tiles: swz_r for row reads only, swz_c for tiles also read down
 // their columns) or 8-byte pieces XOR-swizzled (64-column tiles, t64).
+//
+// Few sequences (segments).  The chunks of a sequence form a chain of about
+// 5 us each, so a launch with fewer (sequence, value head) pairs than the
+// chip's 512 workgroup slots lasts as long as its longest sequence.  A chunk's
+// state update is affine, S^T <- M S^T + N, and so is that of a run of chunks:
+// the sequences are cut into segments, and
+//   1. gdn_chunk_kernel<kState> runs every segment but a sequence's last one
+//      for the states only, once from a zero (first segment: the initial)
+//      state, which gives N, and, past the first segment, once from the identity
+//      without values, which gives M;
+//   2. gdn_combine_kernel chains them, in float32 throughout (fp32 MFMA);
+//   3. gdn_chunk_kernel<kSegment> runs every segment from the state it enters with.
+// Three times the work of the chain, in parallel over all segments.  Chunks
+// start where they do without segments; the states and outputs differ from
+// the chain's as two float32 summation orders do (errors against float64 are
+// the same within 3%).
+#include <algorithm>
+
 #include "nq_device.hpp"
 
 namespace nq {
@@ -71,9 +89,15 @@ struct ChunkArgs {
   const int32_t *cu;
   int H, HV, from_slot, num_seqs;
   float eps, scale;
+  // segments: [max_segs, HV] matrices of 128 x 128 float32
+  float *ws_n;  // N, then the state after the segment, as the pool stores it ([V][K])
+  float *ws_m;  // M [K][K]; of a sequence's first segment, its initial state
+  int max_segs;
 };
+enum { kWhole = 0, kState = 1, kSegment = 2 };
 
 constexpr int kSortSeqs = 64;  // batches up to this size run their longest sequences first
+constexpr int kSegMin = 2;     // chunks per segment, at least
 
 // LDS layout (bytes).
 constexpr int kTile = kC * kD * 2;         // 64 x 128 16-bit values
@@ -195,9 +219,35 @@ __device__ inline u32x4 kt_op(uint32_t base, int o, int s) {
   return cat(lds_load_tr16<0>(base + 8 * o + 32 * 256 * s), lds_load_tr16<0>(base + 8 * o + 32 * 256 * s + 16 * 256));
 }
 
-template <class T>
+// The segments of a launch, the same in every workgroup: sequence `lane` has
+// `segs` of them, of `len` chunks each, numbered from `first`; `total` in all.
+// The length is the shortest with which each pass is one round of resident
+// workgroups: pass 3 runs every segment, pass 1 all but a sequence's last one
+// for N and all but its first and last for M.  At most 64 sequences.  Called
+// by whole waves.
+struct Segments {
+  int len, segs, first, total;
+};
+__device__ inline Segments plan_segments(const ChunkArgs &a, int lane) {
+  const int c = lane < a.num_seqs ? max(1, (a.cu[lane + 1] - a.cu[lane] + kC - 1) / kC) : 0;
+  Segments s;
+  s.len = max(kSegMin, (wave_sum_i32(c) + a.max_segs - 1) / a.max_segs);
+  for (;; ++s.len) {
+    s.segs = (c + s.len - 1) / s.len;  // ends: one segment per sequence fits (host)
+    const int incl = wave_iscan(s.segs);
+    s.first = incl - s.segs;
+    s.total = __builtin_amdgcn_readlane(incl, 63);
+    if (s.total > a.max_segs) continue;
+    if (wave_sum_i32(max(0, s.segs - 1) + max(0, s.segs - 2)) <= a.max_segs) break;
+  }
+  s.len = __builtin_amdgcn_readfirstlane(s.len);
+  return s;
+}
+
+template <class T, int MODE>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_chunk_kernel(
     const ChunkArgs a) {
+  constexpr bool STATE = MODE == kState;  // no q, no outputs
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const uint32_t L = lds_addr(smem);
   const uint32_t LK = L + kOffK, LQ = L + kOffQ, LV = L + kOffV, LA = L + kOffA, LBD = L + kOffB;
@@ -219,7 +269,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   // another, so the longest sequences go first (row y of the grid takes the
   // sequence of rank y by length, ties by index); wave 0 ranks them.
   int n = blockIdx.y;
-  if (a.num_seqs <= kSortSeqs) {
+  int seg = 0, n_segs = 1, seg_len = 0;
+  if constexpr (MODE != kWhole) {
+    const int lane = tid0 & 63;
+    const Segments sg = plan_segments(a, lane);
+    if (static_cast<int>(blockIdx.y) >= sg.total) return;
+    n = __builtin_ctzll(__builtin_amdgcn_ballot_w64(sg.first + sg.segs > static_cast<int>(blockIdx.y)));
+    n = __builtin_amdgcn_readfirstlane(n);
+    seg = static_cast<int>(blockIdx.y) - __builtin_amdgcn_readlane(sg.first, n);
+    n_segs = __builtin_amdgcn_readlane(sg.segs, n);
+    seg_len = sg.len;
+    if (STATE && (seg == n_segs - 1 || (blockIdx.z == 1 && seg == 0))) return;
+  } else if (a.num_seqs <= kSortSeqs) {
     if (wave == 0) {
       const int lane = tid0 & 63;
       const int len = lane < a.num_seqs ? a.cu[lane + 1] - a.cu[lane] : -1;
@@ -238,7 +299,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     lds_sync();  // read by every wave before the region is reused
   }
   const int h = hv / (a.HV / a.H);
-  const int t0 = a.cu[n], t1 = a.cu[n + 1];
+  int t0 = a.cu[n], t1 = a.cu[n + 1];
+  if constexpr (MODE != kWhole) {
+    t0 += seg * seg_len * kC;
+    if (seg < n_segs - 1) t1 = t0 + seg_len * kC;
+  }
+  const bool with_v = !(STATE && blockIdx.z == 1);  // M: no values
   const int slot = a.idx[n];
   const bool has = slot >= 0 && slot < a.num_slots;
   float *st = has ? a.state + (static_cast<int64_t>(slot) * a.HV + hv) * kD * kD : nullptr;
@@ -251,14 +317,34 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   // 32 (kb / 2) + 8 (l / 16) + 4 (kb % 2) + r, value column 32 wave + 16 hf + l % 16.
   const int m0 = tid0 & 15, g0 = (tid0 >> 4) & 3;
   f32x4 S[8][2];
-  auto state_at = [&](int kb, int hf) {
-    return reinterpret_cast<f32x4 *>(st + (32 * wave + 16 * hf + m0) * kD + 32 * (kb >> 1) + 8 * g0 + 4 * (kb & 1));
+  auto state_at = [&](float *base, int kb, int hf) {
+    return reinterpret_cast<f32x4 *>(base + (32 * wave + 16 * hf + m0) * kD + 32 * (kb >> 1) + 8 * g0 + 4 * (kb & 1));
   };
-  if (has && a.from_slot) {
+  // matrix of segment number `no` of this head
+  auto seg_mat = [&](float *ws, int no) { return ws + (static_cast<int64_t>(no) * a.HV + hv) * kD * kD; };
+  float *from = has && a.from_slot ? st : nullptr;
+  if constexpr (STATE) {
+    if (seg > 0) from = nullptr;
+  } else if constexpr (MODE == kSegment) {
+    // A later segment starts where the chain of step 2 arrived.  The first of
+    // several starts from that step's copy of the initial state: the slot
+    // itself takes the final state from another workgroup of this launch.
+    if (seg > 0) from = seg_mat(a.ws_n, blockIdx.y - 1);
+    else if (n_segs > 1 && from) from = seg_mat(a.ws_m, blockIdx.y);
+  }
+  if (from) {
 #pragma unroll
     for (int kb = 0; kb < 8; ++kb)
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf) S[kb][hf] = *state_at(kb, hf);
+      for (int hf = 0; hf < 2; ++hf) S[kb][hf] = *state_at(from, kb, hf);
+  } else if (!with_v) {  // the identity
+#pragma unroll
+    for (int kb = 0; kb < 8; ++kb)
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          S[kb][hf][r] = 32 * (kb >> 1) + 8 * g0 + 4 * (kb & 1) + r == 32 * wave + 16 * hf + m0 ? 1.f : 0.f;
   } else {
 #pragma unroll
     for (int kb = 0; kb < 8; ++kb)
@@ -281,7 +367,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int col2 = (32 * e + 8 * j) * 2;
-      qv[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rq, r * static_cast<int>(a.q_rs) + col2, 0, 0));
+      if constexpr (!STATE)
+        qv[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rq, r * static_cast<int>(a.q_rs) + col2, 0, 0));
       kv[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, r * static_cast<int>(a.k_rs) + col2, 0, 0));
     }
   };
@@ -306,6 +393,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   // (waves 0 and 1: q rows 0-31 and 32-63; waves 2 and 3: the same of k).
   // Rows past the sequence fall outside the descriptor.
   auto warm = [&](int c0, int tid) {
+    if (STATE && wave < 2) return;
     const int rows = min(kC, t1 - c0);
     const uint8_t *src = wave < 2 ? a.q : a.k;
     const int64_t rs = wave < 2 ? a.q_rs : a.k_rs;
@@ -355,7 +443,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     fetch(t0, tid0);
     // P's blocks (0, 1) and (2, 3), read by O += P D and never written
     // otherwise: zero once
-    if (wave < 2) lds_store_b64(t64(L + kOffP, 32 * wave + (tid0 & 15), 4 * (2 * wave + 1) + ((tid0 >> 4) & 3)), u32x2{0u, 0u});
+    if (!STATE && wave < 2) lds_store_b64(t64(L + kOffP, 32 * wave + (tid0 & 15), 4 * (2 * wave + 1) + ((tid0 >> 4) & 3)), u32x2{0u, 0u});
   }
   // Per-lane LDS addresses of the operand reads, formed once: the tile
   // swizzles depend only on a row's low four bits, so every block, k-step or
@@ -403,20 +491,22 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       float sq0 = 0.f, sq1 = 0.f, sk0 = 0.f, sk1 = 0.f;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        sq0 = dot2<T>(qv[j][0], qv[j][0], dot2<T>(qv[j][1], qv[j][1], sq0));
-        sq1 = dot2<T>(qv[j][2], qv[j][2], dot2<T>(qv[j][3], qv[j][3], sq1));
+        if constexpr (!STATE) {
+          sq0 = dot2<T>(qv[j][0], qv[j][0], dot2<T>(qv[j][1], qv[j][1], sq0));
+          sq1 = dot2<T>(qv[j][2], qv[j][2], dot2<T>(qv[j][3], qv[j][3], sq1));
+        }
         sk0 = dot2<T>(kv[j][0], kv[j][0], dot2<T>(kv[j][1], kv[j][1], sk0));
         sk1 = dot2<T>(kv[j][2], kv[j][2], dot2<T>(kv[j][3], kv[j][3], sk1));
       }
       const float sq = sum4(sq0 + sq1), sk = sum4(sk0 + sk1);
       if (e == 0) {
-        stf(LRQ + 4 * r, a.scale * __builtin_amdgcn_rsqf(sq + a.eps));
+        if constexpr (!STATE) stf(LRQ + 4 * r, a.scale * __builtin_amdgcn_rsqf(sq + a.eps));
         stf(LRK + 4 * r, __builtin_amdgcn_rsqf(sk + a.eps));
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int chunk = 4 * e + j;
-        lds_store_b128(a128(LQ, r, chunk, false), qv[j]);
+        if constexpr (!STATE) lds_store_b128(a128(LQ, r, chunk, false), qv[j]);
         lds_store_b128(a128(LK, r, chunk, true), kv[j]);
       }
     }
@@ -424,7 +514,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     // chunk's reads ended before its final barrier); issued after q and k are
     // consumed, so that the compiler's waits for those do not also wait for
     // these copies.  Completed by the vmcnt(0) before the barrier ahead of Z.
-    copy_v(c0, tid);
+    if (with_v) copy_v(c0, tid);
     if (c0 + kC < t1) copy_gates(c0 + kC, gset ^ 1, tid);
     lds_sync();
 
@@ -443,7 +533,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       const int i = 16 * I + m, jb = 16 * J + 4 * g;
       const float Gi = ldf(LG + 4 * i);
       fa = ldf(LB + 4 * i) * ldf(LRK + 4 * i);
-      fp = ldf(LRQ + 4 * i);
+      fp = STATE ? 0.f : ldf(LRQ + 4 * i);
       const f32x4 Gj = ldf4(LG + 4 * jb), rkj = ldf4(LRK + 4 * jb);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
@@ -458,21 +548,23 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       for (int s = 0; s < 4; ++s) {
         kj[s] = lds_load_b128<0>(bK[s] + 16 * 256 * J);
         ki[s] = lds_load_b128<0>(bK[s] + 16 * 256 * I);
-        qi[s] = lds_load_b128<0>(bQ[s] + 16 * 256 * I);
+        if constexpr (!STATE) qi[s] = lds_load_b128<0>(bQ[s] + 16 * 256 * I);
       }
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         ca = T::mfma16x16x32(kj[s], ki[s], ca);
-        cp = T::mfma16x16x32(kj[s], qi[s], cp);
+        if constexpr (!STATE) cp = T::mfma16x16x32(kj[s], qi[s], cp);
       }
       f32x4 dec;
       float fa, fp;
       decay(I, J, dec, fa, fp);
       lds_store_b64(bT[J] + 16 * 128 * I, pack4<T>(-(fa * dec * ca)));                 // A: row 16 I + m, piece 4 J + g
-      lds_store_b64(bT[J] + (kOffP - kOffA) + 16 * 128 * I, pack4<T>(fp * dec * cp));  // P
+      if constexpr (!STATE)
+        lds_store_b64(bT[J] + (kOffP - kOffA) + 16 * 128 * I, pack4<T>(fp * dec * cp));  // P
     };
     // P^T of the diagonal block I: operands K_I, Q_I
     auto diag_p_job = [&](int I) {
+      if constexpr (STATE) return;
       f32x4 cp = f32x4{0.f, 0.f, 0.f, 0.f};
       u32x4 ki[4], qi[4];
 #pragma unroll
@@ -583,7 +675,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb) {
       kr[mb] = lds_load_b128<0>(bK[0] + 16 * 256 * mb);
-      qr[mb] = lds_load_b128<0>(bQ[0] + 16 * 256 * mb);
+      if constexpr (!STATE) qr[mb] = lds_load_b128<0>(bQ[0] + 16 * 256 * mb);
     }
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
@@ -594,11 +686,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
           Y[mb][hf] = T::mfma16x16x32(kr[mb], sb[hf], Y[mb][hf]);
-          O[mb][hf] = T::mfma16x16x32(qr[mb], sb[hf], O[mb][hf]);
+          if constexpr (!STATE) O[mb][hf] = T::mfma16x16x32(qr[mb], sb[hf], O[mb][hf]);
         }
         if (s < 3) {
           kr[mb] = lds_load_b128<0>(bK[s + 1] + 16 * 256 * mb);
-          qr[mb] = lds_load_b128<0>(bQ[s + 1] + 16 * 256 * mb);
+          if constexpr (!STATE) qr[mb] = lds_load_b128<0>(bQ[s + 1] + 16 * 256 * mb);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -626,7 +718,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
-          const f32x4 vf = unpack2x2<T>(vw[mb][hf][0], vw[mb][hf][1]);
+          f32x4 vf = unpack2x2<T>(vw[mb][hf][0], vw[mb][hf][1]);
+          if (STATE && !with_v) vf = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int r = 0; r < 4; ++r) Y[mb][hf][r] = Bt[mb][r] * (vf[r] - Et[mb][r] * Y[mb][hf][r]);
         }
@@ -678,7 +771,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       }
     }
     // ---- O = diag(exp(G)) Q S^T + P D, stored as 16-bit values.
-    {
+    if constexpr (!STATE) {
 #pragma unroll
       for (int mb = 0; mb < 4; ++mb) {
         const f32x4 e4 = ldf4(LEG + 4 * (16 * mb + 4 * g)) * ldf4(LRQ + 4 * (16 * mb + 4 * g));
@@ -730,15 +823,116 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
     lds_sync();  // the next chunk overwrites K, Q, V, A, P; every read of this chunk's is done
   }
-  if (has) {
+  if (STATE && !with_v) {  // M, row by key
+    float *mat = seg_mat(a.ws_m, blockIdx.y);
 #pragma unroll
     for (int kb = 0; kb < 8; ++kb)
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf) *state_at(kb, hf) = S[kb][hf];
+      for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          mat[(32 * (kb >> 1) + 8 * g0 + 4 * (kb & 1) + r) * kD + 32 * wave + 16 * hf + m0] = S[kb][hf][r];
+    return;
+  }
+  float *to = STATE ? seg_mat(a.ws_n, blockIdx.y) : (has && seg == n_segs - 1 ? st : nullptr);
+  if (to) {
+#pragma unroll
+    for (int kb = 0; kb < 8; ++kb)
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) *state_at(to, kb, hf) = S[kb][hf];
+  }
+}
+
+// Step 2 of the segments: S_0 = N_0, S_i = M_i S_{i-1} + N_i, in place of
+// N_i (what segment i + 1 starts from), and the copy of the initial state.
+// One workgroup per 16 value columns of a (sequence, value head): wave w forms
+// keys 16 w .. +15 of them on v_mfma_f32_16x16x4_f32, whose accumulator rows
+// 4 g + r (lane group g) are the next step's B operand for contraction index
+// 16 w + 4 g + r, so the waves only exchange accumulators (8 KiB a step through
+// LDS).  A chain of dependent steps, about 2 us each (1 us of products; 9
+// segments of one sequence 22 us in all), with the M and N of two segments in
+// flight.  A head's workgroups share its M: grid columns of one head go to one
+// XCD (HV a multiple of 8), whose L2 reads M once; with the columns spread over
+// the XCDs the launch took 26 us, with four waves of 32 keys and one segment in
+// flight 4 us a step.
+constexpr int kCombineThreads = 512;
+__global__ __launch_bounds__(kCombineThreads) __attribute__((amdgpu_waves_per_eu(4))) void gdn_combine_kernel(const ChunkArgs a) {
+  __shared__ __attribute__((aligned(16))) f32x4 xch[2][8][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m = lane & 15, g = lane >> 4;
+  const int col = 16 * blockIdx.y + m, hv = blockIdx.x, n = blockIdx.z;
+  const Segments sg = plan_segments(a, lane);
+  const int n_segs = __builtin_amdgcn_readlane(sg.segs, n), first = __builtin_amdgcn_readlane(sg.first, n);
+  if (n_segs < 2) return;
+  auto mat = [&](float *ws, int i) { return ws + (static_cast<int64_t>(first + i) * a.HV + hv) * kD * kD; };
+  const int at = col * kD + 16 * wave + 4 * g;  // this lane's keys of its column
+  if (a.from_slot) {
+    const int slot = a.idx[n];
+    if (slot >= 0 && slot < a.num_slots)
+      *reinterpret_cast<f32x4 *>(mat(a.ws_m, 0) + at) = *reinterpret_cast<const f32x4 *>(
+          a.state + (static_cast<int64_t>(slot) * a.HV + hv) * kD * kD + at);
+  }
+  if (n_segs < 3) return;
+  struct Step {
+    f32x4 m[8], n;
+  };
+  auto load = [&](int i, Step &s) {
+    if (i >= n_segs - 1) return;
+    s.n = *reinterpret_cast<const f32x4 *>(mat(a.ws_n, i) + at);
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+      s.m[t] = *reinterpret_cast<const f32x4 *>(mat(a.ws_m, i) + (16 * wave + m) * kD + 16 * t + 4 * g);
+  };
+  f32x4 sb[8];
+#pragma unroll
+  for (int b = 0; b < 8; ++b)
+    sb[b] = *reinterpret_cast<const f32x4 *>(mat(a.ws_n, 0) + col * kD + 16 * b + 4 * g);
+  Step s0, s1;
+  load(1, s0);
+  load(2, s1);
+  auto step = [&](int i, Step &s) {
+    f32x4 acc[2] = {s.n, f32x4{0.f, 0.f, 0.f, 0.f}};  // two sums shorten the dependent chain
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        acc[r & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(s.m[t][r], sb[t][r], acc[r & 1], 0, 0, 0);
+    const f32x4 v = acc[0] + acc[1];
+    load(i + 2, s);
+    *reinterpret_cast<f32x4 *>(mat(a.ws_n, i) + at) = v;
+    xch[i & 1][wave][lane] = v;
+    lds_sync();  // two buffers: the next step's writes go to the other one
+#pragma unroll
+    for (int t = 0; t < 8; ++t) sb[t] = xch[i & 1][t][lane];
+  };
+  for (int i = 1; i < n_segs - 1; i += 2) {
+    step(i, s0);
+    if (i + 1 >= n_segs - 1) break;
+    step(i + 1, s1);
   }
 }
 
 }  // namespace
+
+// Segments a launch may use at most (0: it runs its sequences whole): one per
+// resident workgroup and value head.  With x the share of the resident
+// workgroups that whole sequences fill, segments win from about 7 + 768 x^2
+// chunks per sequence on (x up to 1/4): the chain gets shorter by the free
+// share, the work is done two and a half times.  Measured, delta rule only,
+// sequences of equal length, whole -> segments: x = 1/16: 10 chunks 53 -> 49.5
+// us, 16 81 -> 58, 63 306 -> 128; x = 1/8: 10 chunks 55 -> 66, 16 83 -> 75, 40
+// 196 -> 140; x = 3/16: 25 chunks 126 -> 126, 40 195 -> 162, 63 310 -> 245; x =
+// 1/4: 40 chunks 195 -> 205, 63 317 -> 303.  Uneven lengths move each in the
+// segments' favour.  With the convolution and the norm: 3 sequences of
+// 2352-3699 tokens at 32 value heads 387 -> 304, one of 8000 693 -> 294 (8 value
+// heads: 641 -> 174).
+int gdn_max_segments(int num_seqs, int64_t total_tokens, int HV) {
+  const int slots = 2 * device_cus();
+  const double x = static_cast<double>(num_seqs) * HV / slots;
+  if (num_seqs > kSortSeqs || x > 0.25 || total_tokens < num_seqs * kC * (7.0 + 768.0 * x * x)) return 0;
+  return slots / HV;
+}
+int64_t gdn_segment_bytes(int max_segs, int HV) { return 2LL * max_segs * HV * kD * kD * 4; }
 
 // Launches the chunked prefill over GdnArgs-style arguments (see
 // nq_gdn_prefill in gdn_decode.hip, which validates them).
@@ -746,7 +940,7 @@ int launch_gdn_chunk_prefill(const void *q, int64_t q_rs, const void *k, int64_t
                              const void *a, int64_t a_rs, const void *b, int64_t b_rs, const float *A_log,
                              const float *dt_bias, const int32_t *cu, int num_seqs, float *state,
                              const int32_t *idx, int64_t num_slots, int from_slot, void *out, int64_t o_rs, int H,
-                             int HV, int dtype, hipStream_t s) {
+                             int HV, int dtype, int64_t total_tokens, void *ws, int64_t ws_bytes, hipStream_t s) {
   ChunkArgs c{};
   c.q = static_cast<const uint8_t *>(q);
   c.k = static_cast<const uint8_t *>(k);
@@ -772,11 +966,26 @@ int launch_gdn_chunk_prefill(const void *q, int64_t q_rs, const void *k, int64_t
   c.from_slot = from_slot;
   c.eps = 1e-6f;
   c.scale = 1.0f / sqrtf(static_cast<float>(kD));
+  c.max_segs = gdn_max_segments(num_seqs, total_tokens, HV);
+  if (ws && c.max_segs > 0 && ws_bytes >= gdn_segment_bytes(c.max_segs, HV)) {
+    c.ws_n = static_cast<float *>(ws);
+    c.ws_m = c.ws_n + static_cast<int64_t>(c.max_segs) * HV * kD * kD;
+    auto *pass1 = dtype == NQ_BF16 ? gdn_chunk_kernel<BF16, kState> : gdn_chunk_kernel<F16, kState>;
+    auto *pass3 = dtype == NQ_BF16 ? gdn_chunk_kernel<BF16, kSegment> : gdn_chunk_kernel<F16, kSegment>;
+    pass1<<<dim3(HV, c.max_segs, 2), kThreads, kLds, s>>>(c);
+    int rc = check_launch("gdn_prefill(segment states)");
+    if (rc != NQ_OK) return rc;
+    gdn_combine_kernel<<<dim3(HV, kD / 16, num_seqs), kCombineThreads, 0, s>>>(c);
+    rc = check_launch("gdn_prefill(combine)");
+    if (rc != NQ_OK) return rc;
+    pass3<<<dim3(HV, c.max_segs), kThreads, kLds, s>>>(c);
+    return check_launch("gdn_prefill(segments)");
+  }
   dim3 grid(HV, num_seqs);
   if (dtype == NQ_BF16)
-    gdn_chunk_kernel<BF16><<<grid, kThreads, kLds, s>>>(c);
+    gdn_chunk_kernel<BF16, kWhole><<<grid, kThreads, kLds, s>>>(c);
   else
-    gdn_chunk_kernel<F16><<<grid, kThreads, kLds, s>>>(c);
+    gdn_chunk_kernel<F16, kWhole><<<grid, kThreads, kLds, s>>>(c);
   return check_launch("gdn_prefill");
 }
 

@@ -37,7 +37,9 @@ int launch_gdn_chunk_prefill(const void *q, int64_t q_rs, const void *k, int64_t
                              const void *a, int64_t a_rs, const void *b, int64_t b_rs, const float *A_log,
                              const float *dt_bias, const int32_t *cu, int num_seqs, float *state,
                              const int32_t *idx, int64_t num_slots, int from_slot, void *out, int64_t o_rs, int H,
-                             int HV, int dtype, hipStream_t s);
+                             int HV, int dtype, int64_t total_tokens, void *ws, int64_t ws_bytes, hipStream_t s);
+int gdn_max_segments(int num_seqs, int64_t total_tokens, int HV);
+int64_t gdn_segment_bytes(int max_segs, int HV);
 namespace {
 
 constexpr int kThreads = 64;
@@ -289,13 +291,13 @@ extern "C" int nq_gdn_decode(const void *q, int64_t q_row_stride, const void *k,
   return check_launch("gdn_decode");
 }
 
-extern "C" int nq_gdn_prefill(const void *q, int64_t q_row_stride, const void *k, int64_t k_row_stride,
+static int gdn_prefill_impl(const void *q, int64_t q_row_stride, const void *k, int64_t k_row_stride,
                               const void *v, int64_t v_row_stride, const void *a, int64_t a_row_stride,
                               const void *b, int64_t b_row_stride, const float *A_log, const float *dt_bias,
                               const int32_t *cu_seqlens, int num_seqs, float *state, const int32_t *state_indices,
                               int64_t num_slots, int initial_state_from_slot, void *out, int64_t out_row_stride,
                               int num_k_heads, int num_v_heads, int head_k_dim, int head_v_dim, int dtype,
-                              void *stream) {
+                              int64_t total_tokens, void *workspace, int64_t workspace_bytes, void *stream) {
   if (num_seqs < 0 || num_k_heads <= 0 || num_v_heads <= 0 || num_slots < 0)
     return fail(NQ_EINVAL, "gdn_prefill: bad sizes (seqs=%d heads=%d/%d)", num_seqs, num_k_heads, num_v_heads);
   if (num_v_heads % num_k_heads != 0)
@@ -310,8 +312,41 @@ extern "C" int nq_gdn_prefill(const void *q, int64_t q_row_stride, const void *k
       (q_row_stride * 2) % 16 || (k_row_stride * 2) % 16 || (v_row_stride * 2) % 16 || (out_row_stride * 2) % 16)
     return fail(NQ_EINVAL, "gdn_prefill: state, q/k/v/out rows 16-byte alignment");
   if (num_seqs > 65535 || num_v_heads > 65535) return fail(NQ_EINVAL, "gdn_prefill: grid too large");
+  if (workspace && !aligned(workspace, 256)) return fail(NQ_EINVAL, "gdn_prefill: workspace alignment");
   return launch_gdn_chunk_prefill(q, q_row_stride * 2, k, k_row_stride * 2, v, v_row_stride * 2, a, a_row_stride * 2,
                                   b, b_row_stride * 2, A_log, dt_bias, cu_seqlens, num_seqs, state, state_indices,
                                   num_slots, initial_state_from_slot, out, out_row_stride * 2, num_k_heads, num_v_heads,
-                                  dtype, static_cast<hipStream_t>(stream));
+                                  dtype, total_tokens, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int nq_gdn_prefill(const void *q, int64_t q_row_stride, const void *k, int64_t k_row_stride,
+                              const void *v, int64_t v_row_stride, const void *a, int64_t a_row_stride,
+                              const void *b, int64_t b_row_stride, const float *A_log, const float *dt_bias,
+                              const int32_t *cu_seqlens, int num_seqs, float *state, const int32_t *state_indices,
+                              int64_t num_slots, int initial_state_from_slot, void *out, int64_t out_row_stride,
+                              int num_k_heads, int num_v_heads, int head_k_dim, int head_v_dim, int dtype,
+                              void *stream) {
+  return gdn_prefill_impl(q, q_row_stride, k, k_row_stride, v, v_row_stride, a, a_row_stride, b, b_row_stride, A_log,
+                          dt_bias, cu_seqlens, num_seqs, state, state_indices, num_slots, initial_state_from_slot, out,
+                          out_row_stride, num_k_heads, num_v_heads, head_k_dim, head_v_dim, dtype, 0, nullptr, 0,
+                          stream);
+}
+
+extern "C" int nq_gdn_prefill_split(const void *q, int64_t q_row_stride, const void *k, int64_t k_row_stride,
+                              const void *v, int64_t v_row_stride, const void *a, int64_t a_row_stride,
+                              const void *b, int64_t b_row_stride, const float *A_log, const float *dt_bias,
+                              const int32_t *cu_seqlens, int num_seqs, float *state, const int32_t *state_indices,
+                              int64_t num_slots, int initial_state_from_slot, void *out, int64_t out_row_stride,
+                              int num_k_heads, int num_v_heads, int head_k_dim, int head_v_dim, int dtype,
+                              int64_t total_tokens, void *workspace, int64_t workspace_bytes, void *stream) {
+  return gdn_prefill_impl(q, q_row_stride, k, k_row_stride, v, v_row_stride, a, a_row_stride, b, b_row_stride, A_log,
+                          dt_bias, cu_seqlens, num_seqs, state, state_indices, num_slots, initial_state_from_slot, out,
+                          out_row_stride, num_k_heads, num_v_heads, head_k_dim, head_v_dim, dtype, total_tokens,
+                          workspace, workspace_bytes, stream);
+}
+
+extern "C" int64_t nq_gdn_prefill_workspace_bytes(int num_seqs, int64_t total_tokens, int num_v_heads) {
+  if (num_seqs <= 0 || total_tokens <= 0 || num_v_heads <= 0) return 0;
+  const int segs = gdn_max_segments(num_seqs, total_tokens, num_v_heads);
+  return segs > 0 ? gdn_segment_bytes(segs, num_v_heads) : 0;
 }

@@ -32,6 +32,7 @@ from ._lib import check, dtype_code, lib, ptr, require_cuda, stream_of
 _workspaces: dict[tuple[int, int], torch.Tensor] = {}
 _prefill_queues: dict[tuple[int, int], torch.Tensor] = {}
 _prefill_parts: dict[tuple[int, int], torch.Tensor] = {}
+_gdn_segments: dict[tuple[int, int], torch.Tensor] = {}
 _retired: list[torch.Tensor] = []
 _DEBUG_QUEUE = os.environ.get("NQ_DEBUG_PREFILL_QUEUE", "0") not in ("", "0")
 
@@ -61,14 +62,14 @@ def _grow(table, key, nbytes, dtype, device, zero=False):
 
 def release_workspaces(device=None) -> int:
     """Drop the kernels' per-stream buffers (decode split-K workspaces,
-    prefill queue counters and partial outputs) and every retired buffer, of ``device`` or of
+    prefill queue counters and partial outputs, GDN segment states) and every retired buffer, of ``device`` or of
     all devices; returns how many were dropped.  Only safe once no HIP graph
     captured with them will be replayed again: a replay would write freed
     memory.  Later calls allocate fresh buffers (the prefill counters start
     at zero again)."""
     idx = None if device is None else _key(device)[0]
     n = 0
-    for table in (_workspaces, _prefill_queues, _prefill_parts):
+    for table in (_workspaces, _prefill_queues, _prefill_parts, _gdn_segments):
         for key in [k for k in table if idx is None or k[0] == idx]:
             del table[key]
             n += 1
@@ -493,11 +494,16 @@ def gdn_prefill(query, key, value, a, b, A_log, dt_bias, cu_seqlens, state, stat
     for t, what in ((query, "query"), (key, "key"), (value, "value"), (a2, "a"), (b2, "b")):
         if _overlaps(out, t):
             raise RuntimeError(f"gdn_prefill: out must not overlap {what}")
-    rc = lib().nq_gdn_prefill(ptr(query), query.stride(0), ptr(key), key.stride(0), ptr(value), value.stride(0),
-                              ptr(a2), a2.stride(0), ptr(b2), b2.stride(0), ptr(A_log.contiguous()),
-                              ptr(dt_bias.contiguous()), ptr(cu_seqlens), n, ptr(state), ptr(state_indices),
-                              state.shape[0], 1 if initial_state_from_slot else 0, ptr(out), out.stride(0),
-                              H, HV, K, V, dtype_code(query.dtype), stream_of(query))
+    args = (ptr(query), query.stride(0), ptr(key), key.stride(0), ptr(value), value.stride(0), ptr(a2), a2.stride(0),
+            ptr(b2), b2.stride(0), ptr(A_log.contiguous()), ptr(dt_bias.contiguous()), ptr(cu_seqlens), n, ptr(state),
+            ptr(state_indices), state.shape[0], 1 if initial_state_from_slot else 0, ptr(out), out.stride(0),
+            H, HV, K, V, dtype_code(query.dtype))
+    seg_bytes = lib().nq_gdn_prefill_workspace_bytes(n, T_, HV)
+    if seg_bytes > 0:    # few sequences: cut into segments that run side by side
+        ws = _grow(_gdn_segments, _key(query.device), seg_bytes, torch.uint8, query.device)
+        rc = lib().nq_gdn_prefill_split(*args, T_, ptr(ws), ws.numel(), stream_of(query))
+    else:
+        rc = lib().nq_gdn_prefill(*args, stream_of(query))
     check(rc, "gdn_prefill")
     return out
 

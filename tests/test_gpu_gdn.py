@@ -467,3 +467,51 @@ def test_gdn_prefill_random_sweep(cuda, seed):
     untouched = [sl for sl in range(nseq + 2) if sl not in live]
     for sl in untouched:  # slots no sequence names keep their contents
         assert torch.equal(state_dev[sl], d["state"][sl])
+
+
+@pytest.mark.parametrize("lens,H,HV,kind", [
+    ([1300], 16, 32, "random"),
+    ([64 * 9, 64 * 9 + 1, 64 * 20 - 1], 2, 8, "random"),      # segment and chunk edges
+    ([4000, 0, 65, 40, 1], 4, 8, "random"),                    # one long, empty and short ones
+    ([5000], 2, 4, "random"),                                  # as many segments as they come
+    ([2100, 900], 4, 8, "slow"),                               # little decay and small updates: long memory
+    ([1200, 1200], 8, 8, "f16"),
+    ([1700, 2500, 1400, 3700], 4, 16, "random"),
+], ids=str)
+@pytest.mark.parametrize("from_slot", [False, True])
+def test_gdn_prefill_segments(cuda, lens, H, HV, kind, from_slot, monkeypatch):
+    """Few sequences run as segments (states, float32 chaining, outputs):
+    outputs and final states against the float64 chunked form, and no further
+    from it than the same launch with whole sequences."""
+    n, slots = len(lens), len(lens) + 2
+    c = _prefill_inputs(lens, H, HV, seed=sum(lens), slots=slots,
+                        dtype=torch.float16 if kind == "f16" else torch.bfloat16)
+    if kind == "slow":
+        c["A_log"][:] = -6.0
+        c["b"] -= 3.0
+    idx = torch.randperm(slots, generator=torch.Generator().manual_seed(n))[:n].to(torch.int32)
+    skip = n > 3
+    if skip:
+        idx[2] = -1    # keeps no state and starts from zero
+    d = {k: v.to(cuda) for k, v in c.items()}
+    lib = kernels.lib()
+    assert lib.nq_gdn_prefill_workspace_bytes(n, sum(lens), HV) > 0
+    ref_state = d["state"].double().clone()
+    ref = gdn.gdn_prefill_chunked(d["q"], d["k"], d["v"], d["a"], d["b"], d["A_log"], d["dt"], c["cu"], ref_state,
+                                  idx, from_slot=from_slot)
+    live = [i for i in idx.tolist() if i >= 0]
+    off = {}
+    for how in ("segments", "whole"):
+        if how == "whole":
+            monkeypatch.setattr(lib, "nq_gdn_prefill_workspace_bytes", lambda *a: 0)
+        state = d["state"].clone()
+        out = kernels.gdn_prefill(d["q"], d["k"], d["v"], d["a"], d["b"], d["A_log"], d["dt"], d["cu"], state,
+                                  idx.to(cuda), initial_state_from_slot=from_slot)
+        torch.cuda.synchronize()
+        _prefill_close(out.double().cpu().numpy(), ref.cpu().numpy(), state.double().cpu().numpy()[live],
+                       ref_state.cpu().numpy()[live])
+        untouched = [i for i in range(slots) if i not in live]
+        assert torch.equal(state[untouched], d["state"][untouched])
+        off[how] = [float((x.double() - y).norm() / y.norm()) for x, y in ((out, ref), (state[live], ref_state[live]))]
+    print(f"[gdn] {lens} {kind}: error of outputs and states {off}", flush=True)
+    assert all(s <= 1.1 * w for s, w in zip(off["segments"], off["whole"]))
