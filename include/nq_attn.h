@@ -204,6 +204,34 @@ int nq_paged_decode_store(const void *q, int64_t q_batch_stride, int64_t q_head_
                           void *stream);
 
 /*
+ * The decode step of a small batch in one launch: nq_paged_decode_store, with
+ * k_new (no store when null) and gate optional, whose splits are merged by the
+ * workgroup of each (sequence, kv head) that finishes last.  counters: 64
+ * bytes of device memory per (sequence, kv head), 64-byte aligned, zero before
+ * the first call that uses them; every completed call leaves them zero.  Calls that overlap may
+ * share neither them nor the workspace.  num_splits and split_tokens as
+ * nq_decode_config gives them (any plan that nq_paged_decode accepts is).
+ */
+int nq_paged_decode_fused(const void *q, int64_t q_batch_stride, int64_t q_head_stride,
+                          void *k_cache, void *v_cache, const int32_t *block_tables, int64_t bt_stride,
+                          int max_blocks_per_seq, const int32_t *context_lens, const void *k_new,
+                          int64_t k_new_row_stride, const void *v_new, int64_t v_new_row_stride,
+                          const int32_t *slot_mapping, int new_dtype, void *out,
+                          int64_t out_batch_stride, int64_t out_head_stride, int batch,
+                          int num_q_heads, int num_kv_heads, int head_dim, int block_size,
+                          int64_t num_blocks, float softmax_scale, int num_splits, int split_tokens,
+                          void *workspace, int64_t workspace_bytes, int q_dtype, int kv_dtype,
+                          const float *k_scale, const float *v_scale, const void *gate,
+                          int64_t gate_batch_stride, int64_t gate_head_stride, void *counters,
+                          int64_t counter_bytes, void *stream);
+
+/* How a decode of these sizes runs best, in config[4]: bytes of counters of
+ * nq_paged_decode_fused (0: nq_paged_decode or nq_paged_decode_store instead),
+ * num_splits, split_tokens, bytes of workspace.  Host-known sizes only. */
+int nq_decode_config(int batch, int num_q_heads, int num_kv_heads, int head_dim, int max_blocks_per_seq,
+                     int block_size, int kv_dtype, int64_t *config);
+
+/*
  * nq_paged_decode without a caller workspace, for callers that cannot
  * allocate (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  No counterpart in the reference: it is
@@ -211,7 +239,9 @@ int nq_paged_decode_store(const void *q, int64_t q_batch_stride, int64_t q_head_
  * NQ_DECODE_NOALLOC_SCRATCH_BYTES per device, which each device holds until
  * the process ends.  It calls no allocating routine; the array's address is
  * looked up (hipGetSymbolAddress) on the first call on each device.
- * Every other argument is as for nq_paged_decode.  A plan whose splits
+ * Every other argument is as for nq_paged_decode.  Sizes that
+ * nq_decode_config runs in one launch run that kernel, with its own plan, and
+ * with its counters in the array, zeroed by a launch before it.  A plan whose splits
  * were grown past the table (nq_decode_plan sizes a stream-K workspace that
  * way) runs with the splits that cover the table when the grown plan's
  * nq_decode_workspace_bytes exceeds the array; only a plan whose covering

@@ -56,6 +56,7 @@ struct DecodeArgs {
   float *ws_o;         // split-K [B, Hq, S, D]; stream-K [W, 2, Hq, D]
   float *ws_lse;       // split-K [B, Hq, S]; stream-K [W, 2, Hq]
   int2 *sk_bnd;        // stream-K: [W] range starts (sequence, token)
+  unsigned *counters;  // one-launch merge: [B, Hkv], zero between launches
   uint8_t *ws_raw;     // the caller's workspace and its size
   int64_t ws_bytes;
   int Hq, Hkv, G, block_size;
@@ -284,13 +285,18 @@ struct DecodeWave {
 };
 
 // The work of one wave on one piece of a sequence: kv head kvh of sequence
-// b over tokens [t_begin, t_end) (t_begin % 32 == 0, at most 63 blocks).  A
-// piece that is the whole context (single) writes `out`; any other writes
-// its heads' normalised partial O and log2-sum-exp to workspace row
-// ws_row + head * ws_head_stride, for a merge pass.
-template <class T, bool FP8, int D, int DEPTH>
+// b over tokens [t_begin, t_end) (t_begin % 32 == 0, at most 63 blocks).
+// STRIDE 1: the wave takes all 32-token steps; a piece that is the whole
+// context (single) writes `out`; any other writes its heads' normalised
+// partial O and log2-sum-exp to workspace row ws_row + head * ws_head_stride,
+// for a merge pass.  STRIDE > 1: the wave takes steps first, first + STRIDE, ...
+// of a piece shared with other waves, and leaves its heads' maxima (log2
+// domain) and row sums in wm and wl and its O [head][dim] in its tile.
+template <class T, bool FP8, int D, int DEPTH, int STRIDE = 1>
 __device__ __forceinline__ void decode_piece(const DecodeArgs &a, uint8_t *tile, int b, int kvh, int t_begin,
-                                             int t_end, bool single, int64_t ws_row, int64_t ws_head_stride) {
+                                             int t_end, bool single, int64_t ws_row, int64_t ws_head_stride,
+                                             int first = 0, float *wm = nullptr, float *wl = nullptr) {
+  constexpr int kNext = kStep * STRIDE;  // tokens to the wave's next step
   using W = DecodeWave<T, FP8, D>;
   using Gm = Geo<D, FP8>;
   const int lane = threadIdx.x & 63;
@@ -343,7 +349,7 @@ __device__ __forceinline__ void decode_piece(const DecodeArgs &a, uint8_t *tile,
   int64_t rows[DEPTH];
 #pragma unroll
   for (int d = 0; d < DEPTH; ++d) {
-    const int td = t_begin + d * kStep;
+    const int td = t_begin + first * kStep + d * kNext;
     rows[d] = td < t_end ? W::step_row(a, bt_lane, first_blk, td) : -1;
     W::load(a.k_cache, a, rows[d], td, t_end, voff0, kraw[d]);
     W::load(a.v_cache, a, rows[d], td, t_end, voff0, vraw[d]);
@@ -357,7 +363,7 @@ __device__ __forceinline__ void decode_piece(const DecodeArgs &a, uint8_t *tile,
   // One 32-token step on register set (kr, vr) holding tokens t0..t0+31 of
   // cache row `row`; returns the row of the step that refilled the set.
   auto step = [&](int t0, int64_t row, u32x4 (&kr)[Gm::RAW], u32x4 (&vr)[Gm::RAW]) -> int64_t {
-    const int tn = t0 + DEPTH * kStep;
+    const int tn = t0 + DEPTH * kNext;
     const int64_t rown = (tn < t_end) ? W::step_row(a, bt_lane, first_blk, tn) : -1;
     wave_lds_sync();  // the previous step's V^T reads are issued before the tile is overwritten
     W::stage(tile, kr, lane);
@@ -411,16 +417,27 @@ __device__ __forceinline__ void decode_piece(const DecodeArgs &a, uint8_t *tile,
     return rown;
   };
 
-  for (int t0 = t_begin; t0 < t_end; t0 += DEPTH * kStep) {
+  for (int t0 = t_begin + first * kStep; t0 < t_end; t0 += DEPTH * kNext) {
     rows[0] = step(t0, rows[0], kraw[0], vraw[0]);
     if constexpr (DEPTH > 1) {
-      if (t0 + kStep >= t_end) break;
-      rows[1] = step(t0 + kStep, rows[1], kraw[1], vraw[1]);
+      if (t0 + kNext >= t_end) break;
+      rows[1] = step(t0 + kNext, rows[1], kraw[1], vraw[1]);
     }
   }
 
   // ---- epilogue: lane (m, g) holds O^T[16j + 4g + r][head m]
   const float L = sum32(sum16(l_run));
+  if constexpr (STRIDE > 1) {
+    if (g == 0) {
+      wm[m] = m_run;
+      wl[m] = L;
+    }
+    wave_lds_sync();  // the last step's V^T reads are issued before the tile is overwritten
+    if (m < G)
+#pragma unroll
+      for (int j = 0; j < Gm::NJ; ++j) *reinterpret_cast<f32x4 *>(tile + (m * D + 16 * j + 4 * g) * 4) = o[j];
+    return;
+  }
   if (m >= G) return;
   const int head = kvh * G + m;
   const float inv = (L > 0.f) ? vscale / L : 0.f;
@@ -493,6 +510,254 @@ void paged_decode_kernel(const DecodeArgs a) {
   decode_piece<T, FP8, D, DEPTH>(a, smem + wave * DecodeWave<T, FP8, D>::LDS_PER_WAVE_B, b, kvh, t_begin, t_end,
                                  ctx <= a.split_tokens,
                                  static_cast<int64_t>(b) * a.Hq * a.num_splits + split, a.num_splits);
+}
+
+// Partials of one (sequence, head) -- pieces 0 .. n - 1 -- merged by GR groups
+// of kPer = D / 4 threads: group r takes pieces r, r + GR, ..., loading up to
+// kMergeUnroll of them at once (one round trip for kMergeUnroll * GR pieces),
+// and the groups' sums are combined through LDS.  row(i): workspace row of
+// piece i, or -1 for a piece without tokens.  An empty piece's partials
+// (lse -inf) are never used: they may be stale.  The threads of group 0
+// return true and the merged values in acc; `later` tells every thread
+// whether a piece past the first has tokens.
+//
+// A piece per 32-128 tokens keeps a small batch's main kernel short but
+// leaves up to a few hundred pieces per head.  One thread group that walks
+// them (8 sequences of up to 3000 tokens at head_dim 256, 110 pieces) took
+// 71 us, against 13 us for the attention itself; MERGED
+constexpr int kMergeUnroll = 8;
+// Running (maximum, weight sum, weighted sum) of pieces first, first + step, ...
+// of n, UNROLL of them in flight; `any`: a piece past the first has tokens.
+// SHARED: the pieces were written in this launch, by workgroups of any XCD:
+// read by device-scope atomic loads.
+__device__ __forceinline__ float load_shared(const float *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ f32x4 load_shared4(const float *p) {
+  const uint64_t *q = reinterpret_cast<const uint64_t *>(p);
+  const uint64_t lo = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const uint64_t hi = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return f32x4{u2f(static_cast<uint32_t>(lo)), u2f(static_cast<uint32_t>(lo >> 32)), u2f(static_cast<uint32_t>(hi)),
+               u2f(static_cast<uint32_t>(hi >> 32))};
+}
+__device__ __forceinline__ void store_shared4(float *p, const f32x4 &v) {
+  uint64_t *q = reinterpret_cast<uint64_t *>(p);
+  const uint64_t lo = f2u(v[0]) | (static_cast<uint64_t>(f2u(v[1])) << 32);
+  const uint64_t hi = f2u(v[2]) | (static_cast<uint64_t>(f2u(v[3])) << 32);
+  __hip_atomic_store(q, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(q + 1, hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <int D, int UNROLL, bool SHARED, class Row>
+__device__ __forceinline__ void merge_loop(const DecodeArgs &a, int first, int step, int n, Row row, int d4, float &M, float &W,
+                                           f32x4 &acc, bool &any) {
+  M = kNegInf;
+  W = 0.f;
+  acc = f32x4{0, 0, 0, 0};
+  any = false;
+  // The pieces in chunks, each chunk's loads issued together; the running
+  // maximum rescales the earlier chunks' sums.
+#pragma unroll 1
+  for (int c0 = first; c0 < n; c0 += UNROLL * step) {
+    float l[UNROLL];
+    f32x4 p[UNROLL];
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      const int i = c0 + u * step;
+      l[u] = kNegInf;
+      if (i < n) {
+        const int64_t w = row(i);
+        if (w >= 0) {
+          const float *po = a.ws_o + w * D + 4 * d4;
+          if constexpr (SHARED) {
+            l[u] = load_shared(a.ws_lse + w);
+            p[u] = load_shared4(po);
+          } else {
+            l[u] = a.ws_lse[w];
+            p[u] = *reinterpret_cast<const f32x4 *>(po);
+          }
+        }
+      }
+    }
+    float mc = kNegInf;
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      if (c0 + u * step >= 1) any |= l[u] != kNegInf;
+      mc = fmaxf(mc, l[u]);
+    }
+    if (mc == kNegInf) continue;  // every piece of the chunk is empty
+    const float mn = fmaxf(M, mc);
+    if (M != kNegInf) {
+      const float f = __builtin_amdgcn_exp2f(M - mn);
+      W *= f;
+      acc *= f;
+    }
+    M = mn;
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u)
+      if (l[u] != kNegInf) {
+        const float w = __builtin_amdgcn_exp2f(l[u] - M);
+        W += w;
+        acc += p[u] * w;
+      }
+  }
+}
+template <int D, int GR, class Row>
+__device__ __forceinline__ bool merge_pieces(const DecodeArgs &a, int n, Row row, bool &later, f32x4 &acc) {
+  constexpr int kPer = D / 4;
+  const int d4 = threadIdx.x % kPer, r = GR == 1 ? 0 : threadIdx.x / kPer;
+  float W, M;
+  bool any;
+  merge_loop<D, kMergeUnroll, false>(a, r, GR, n, row, d4, M, W, acc, any);
+  if constexpr (GR > 1) {
+    __shared__ __attribute__((aligned(16))) float part[GR][D];
+    __shared__ float part_m[GR], part_w[GR];
+    *reinterpret_cast<f32x4 *>(&part[r][4 * d4]) = acc;
+    if (d4 == 0) {
+      part_m[r] = M;
+      part_w[r] = W;
+    }
+    any = __syncthreads_or(any);
+    if (r == 0) {
+      float mx = part_m[0];
+#pragma unroll
+      for (int u = 1; u < GR; ++u) mx = fmaxf(mx, part_m[u]);
+      W = 0.f;
+      acc = f32x4{0, 0, 0, 0};
+      if (mx != kNegInf)
+#pragma unroll
+        for (int u = 0; u < GR; ++u) {
+          const float f = __builtin_amdgcn_exp2f(part_m[u] - mx);  // 0 for a group without pieces
+          W += part_w[u] * f;
+          acc += *reinterpret_cast<const f32x4 *>(&part[u][4 * d4]) * f;
+        }
+    }
+  }
+  later = any;
+  acc *= W > 0.f ? 1.0f / W : 0.f;
+  return r == 0;
+}
+
+// One merged row piece to the output, gated if the launch is.
+template <class T>
+__device__ __forceinline__ void store_merged(const DecodeArgs &a, int b, int head, int d4, const f32x4 &acc) {
+  uint8_t *op = a.out + b * a.o_bs + head * a.o_hs + d4 * 8;
+  if (a.gate)
+    *reinterpret_cast<u32x2 *>(op) =
+        gate4<T>(acc, *reinterpret_cast<const u32x2 *>(a.gate + b * a.g_bs + head * a.g_hs + d4 * 8));
+  else
+    *reinterpret_cast<u32x2 *>(op) = u32x2{T::pack2(acc[0], acc[1]), T::pack2(acc[2], acc[3])};
+}
+
+// ---------------------------------------------------------------- one launch
+// Small batches (decode_fused_plan): the four waves of a workgroup take the
+// 32-token steps of one (sequence, kv head, split) in turn, so that a split of
+// a few hundred tokens is one or two round trips to memory, and combine their
+// states through LDS.  A sequence of several splits is merged in the same launch
+// by the workgroup that finishes last: each writes its partial, then counts
+// itself with a release / acquire increment (at device scope: the splits of a
+// sequence may run on XCDs whose L2s are not coherent) in counters[b, kvh],
+// which the last one puts back to zero.
+constexpr int kFusedWaves = 4;
+constexpr int kCounterBytes = 64;  // a counter per cache line: increments of one line are served one by one
+template <class T, bool FP8, int D, int DEPTH, int WPE>
+__global__ __launch_bounds__(64 * kFusedWaves) __attribute__((amdgpu_waves_per_eu(WPE)))
+void paged_decode_fused_kernel(const DecodeArgs a) {
+  using Gm = Geo<D, FP8>;
+  using Wv = DecodeWave<T, FP8, D>;
+  constexpr int NW = kFusedWaves, kPer = D / 4;
+  static_assert(16 * D * 4 <= Gm::TILE_B, "a wave's O in its tile");
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  __shared__ float wm[NW][16], wl[NW][16];
+  __shared__ int last;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int kvh = blockIdx.x, split = blockIdx.y, b = blockIdx.z;
+  if (a.k_new && split == 0 && wave == 0) Wv::store_new(a, b, kvh, lane);
+  const int ctx = min(a.context_lens[b], a.max_tokens);
+  const int t_begin = split * a.split_tokens;
+  if (ctx <= 0 || t_begin >= ctx) {
+    if (ctx <= 0 && split == 0 && wave == 0) decode_zero_row<D>(a, b, kvh, lane);
+    return;  // whole workgroup
+  }
+  const int t_end = min(t_begin + a.split_tokens, ctx);
+  uint8_t *tile = smem + wave * Wv::LDS_PER_WAVE_B;
+  decode_piece<T, FP8, D, DEPTH, NW>(a, tile, b, kvh, t_begin, t_end, false, 0, 0, wave, wm[wave], wl[wave]);
+  __syncthreads();
+  const float vscale = FP8 ? a.v_scale[kvh] : 1.0f;
+  const int n_split = (ctx + a.split_tokens - 1) / a.split_tokens;
+  for (int e = threadIdx.x; e < a.G * kPer; e += 64 * NW) {
+    const int h = e / kPer, d4 = e % kPer, head = kvh * a.G + h;
+    float M = wm[0][h];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) M = fmaxf(M, wm[w][h]);
+    const float mu = M == kNegInf ? 0.f : M;
+    float L = 0.f;
+    f32x4 acc{0, 0, 0, 0};
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float f = __builtin_amdgcn_exp2f(wm[w][h] - mu);
+      L += wl[w][h] * f;
+      acc += *reinterpret_cast<const f32x4 *>(smem + w * Wv::LDS_PER_WAVE_B + (h * D + 4 * d4) * 4) * f;
+    }
+    acc *= L > 0.f ? vscale / L : 0.f;
+    if (n_split == 1) {
+      store_merged<T>(a, b, head, d4, acc);
+    } else {
+      const int64_t idx = (static_cast<int64_t>(b) * a.Hq + head) * a.num_splits + split;
+      store_shared4(a.ws_o + idx * D + 4 * d4, acc);
+      if (d4 == 0)
+        __hip_atomic_store(a.ws_lse + idx, L > 0.f ? M + __log2f(L) : kNegInf, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  if (n_split == 1) return;
+  wait_vmcnt<0>();  // this wave's device-scope stores have completed
+  __syncthreads();  // and every other wave's
+  if (threadIdx.x == 0) {
+    unsigned *c = a.counters + (static_cast<int64_t>(b) * a.Hkv + kvh) * (kCounterBytes / 4);
+    const unsigned before = __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    last = before == static_cast<unsigned>(n_split - 1);
+    if (last) __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (!last) return;
+  // The merge: groups of G * D / 4 threads share the splits when several fit
+  // the workgroup, 16 splits in flight in each, and combine through LDS.
+  const int n_el = a.G * kPer, n_grp = max(1, 64 * NW / n_el);
+  float *part = reinterpret_cast<float *>(smem);  // [group][element]: 4 sums, maximum, weight sum
+  for (int e0 = 0; e0 < n_el; e0 += 64 * NW) {
+    const int r = n_grp > 1 ? threadIdx.x / n_el : 0, e = n_grp > 1 ? threadIdx.x % n_el : e0 + threadIdx.x;
+    const int h = e / kPer, d4 = e % kPer, head = kvh * a.G + h;
+    const int64_t base = (static_cast<int64_t>(b) * a.Hq + head) * a.num_splits;
+    float M = kNegInf, W = 0.f;
+    f32x4 acc{0, 0, 0, 0};
+    bool any;
+    if (r < n_grp && e < n_el)
+      merge_loop<D, 16, true>(a, r, n_grp, n_split, [&](int i) { return base + i; }, d4, M, W, acc, any);
+    if (n_grp > 1) {  // one round: n_el <= 128
+      if (r > 0 && r < n_grp) {
+        float *o = part + (r * n_el + e) * 8;
+        *reinterpret_cast<f32x4 *>(o) = acc;
+        o[4] = M;
+        o[5] = W;
+      }
+      __syncthreads();
+      if (r == 0) {
+        for (int u = 1; u < n_grp; ++u) {
+          const float *o = part + (u * n_el + e) * 8;
+          const float mx = fmaxf(M, o[4]);
+          const float mu = mx == kNegInf ? 0.f : mx;
+          const float f0 = __builtin_amdgcn_exp2f(M - mu), f1 = __builtin_amdgcn_exp2f(o[4] - mu);
+          W = W * f0 + o[5] * f1;
+          acc = acc * f0 + *reinterpret_cast<const f32x4 *>(o) * f1;
+          M = mx;
+        }
+      }
+    }
+    if (r == 0 && e < n_el) {
+      acc *= W > 0.f ? 1.0f / W : 0.f;
+      store_merged<T>(a, b, head, d4, acc);
+    }
+  }
 }
 
 // ---------------------------------------------------------------- stream-K
@@ -590,107 +855,6 @@ int env_int(const char *name, int dflt) {
   const char *v = getenv(name);
   if (!v || !*v) return dflt;
   return atoi(v);
-}
-
-// Partials of one (sequence, head) -- pieces 0 .. n - 1 -- merged by GR groups
-// of kPer = D / 4 threads: group r takes pieces r, r + GR, ..., loading up to
-// kMergeUnroll of them at once (one round trip for kMergeUnroll * GR pieces),
-// and the groups' sums are combined through LDS.  row(i): workspace row of
-// piece i, or -1 for a piece without tokens.  An empty piece's partials
-// (lse -inf) are never used: they may be stale.  The threads of group 0
-// return true and the merged values in acc; `later` tells every thread
-// whether a piece past the first has tokens.
-//
-// A piece per 32-128 tokens keeps a small batch's main kernel short but
-// leaves up to a few hundred pieces per head.  One thread group that walks
-// them (8 sequences of up to 3000 tokens at head_dim 256, 110 pieces) took
-// 71 us, against 13 us for the attention itself; MERGED
-constexpr int kMergeUnroll = 8;
-template <int D, int GR, class Row>
-__device__ __forceinline__ bool merge_pieces(const DecodeArgs &a, int n, Row row, bool &later, f32x4 &acc) {
-  constexpr int kPer = D / 4;
-  const int d4 = threadIdx.x % kPer, r = GR == 1 ? 0 : threadIdx.x / kPer;
-  float W = 0.f, M = kNegInf;
-  acc = f32x4{0, 0, 0, 0};
-  bool any = false;  // a piece past the first has tokens
-  // The pieces in chunks, each chunk's loads issued together; the running
-  // maximum rescales the earlier chunks' sums.
-#pragma unroll 1
-  for (int c0 = r; c0 < n; c0 += kMergeUnroll * GR) {
-    float l[kMergeUnroll];
-    f32x4 p[kMergeUnroll];
-#pragma unroll
-    for (int u = 0; u < kMergeUnroll; ++u) {
-      const int i = c0 + u * GR;
-      l[u] = kNegInf;
-      if (i < n) {
-        const int64_t w = row(i);
-        if (w >= 0) {
-          l[u] = a.ws_lse[w];
-          p[u] = *reinterpret_cast<const f32x4 *>(a.ws_o + w * D + 4 * d4);
-        }
-      }
-    }
-    float mc = kNegInf;
-#pragma unroll
-    for (int u = 0; u < kMergeUnroll; ++u) {
-      if (c0 + u * GR >= 1) any |= l[u] != kNegInf;
-      mc = fmaxf(mc, l[u]);
-    }
-    if (mc == kNegInf) continue;  // every piece of the chunk is empty
-    const float mn = fmaxf(M, mc);
-    if (M != kNegInf) {
-      const float f = __builtin_amdgcn_exp2f(M - mn);
-      W *= f;
-      acc *= f;
-    }
-    M = mn;
-#pragma unroll
-    for (int u = 0; u < kMergeUnroll; ++u)
-      if (l[u] != kNegInf) {
-        const float w = __builtin_amdgcn_exp2f(l[u] - M);
-        W += w;
-        acc += p[u] * w;
-      }
-  }
-  if constexpr (GR > 1) {
-    __shared__ __attribute__((aligned(16))) float part[GR][D];
-    __shared__ float part_m[GR], part_w[GR];
-    *reinterpret_cast<f32x4 *>(&part[r][4 * d4]) = acc;
-    if (d4 == 0) {
-      part_m[r] = M;
-      part_w[r] = W;
-    }
-    any = __syncthreads_or(any);
-    if (r == 0) {
-      float mx = part_m[0];
-#pragma unroll
-      for (int u = 1; u < GR; ++u) mx = fmaxf(mx, part_m[u]);
-      W = 0.f;
-      acc = f32x4{0, 0, 0, 0};
-      if (mx != kNegInf)
-#pragma unroll
-        for (int u = 0; u < GR; ++u) {
-          const float f = __builtin_amdgcn_exp2f(part_m[u] - mx);  // 0 for a group without pieces
-          W += part_w[u] * f;
-          acc += *reinterpret_cast<const f32x4 *>(&part[u][4 * d4]) * f;
-        }
-    }
-  }
-  later = any;
-  acc *= W > 0.f ? 1.0f / W : 0.f;
-  return r == 0;
-}
-
-// One merged row piece to the output, gated if the launch is.
-template <class T>
-__device__ __forceinline__ void store_merged(const DecodeArgs &a, int b, int head, int d4, const f32x4 &acc) {
-  uint8_t *op = a.out + b * a.o_bs + head * a.o_hs + d4 * 8;
-  if (a.gate)
-    *reinterpret_cast<u32x2 *>(op) =
-        gate4<T>(acc, *reinterpret_cast<const u32x2 *>(a.gate + b * a.g_bs + head * a.g_hs + d4 * 8));
-  else
-    *reinterpret_cast<u32x2 *>(op) = u32x2{T::pack2(acc[0], acc[1]), T::pack2(acc[2], acc[3])};
 }
 
 // Threads and (sequence, head) pairs of a merge workgroup with GR groups per
@@ -888,6 +1052,13 @@ struct DecodeLaunch {
   hipStream_t s;
   template <int H, int DP, int WP>
   int run() const {
+    if (a.counters) {
+      constexpr size_t flds = static_cast<size_t>(kFusedWaves) * DecodeWave<T, FP8, D>::LDS_PER_WAVE_B;
+      const int64_t covers = (static_cast<int64_t>(a.max_tokens) + a.split_tokens - 1) / a.split_tokens;
+      paged_decode_fused_kernel<T, FP8, D, DP, (D == 256 ? 1 : 2)>
+          <<<dim3(a.Hkv, static_cast<int>(covers), batch), 64 * kFusedWaves, flds, s>>>(a);
+      return check_launch("paged_decode(one launch)");
+    }
     const int groups = (a.Hkv + H - 1) / H;
     const size_t lds = static_cast<size_t>(H) * DecodeWave<T, FP8, D>::LDS_PER_WAVE_B;
     auto *kern = paged_decode_sk_kernel<T, FP8, D, H, DP, (WP > 2 ? 2 : WP)>;
@@ -1085,7 +1256,7 @@ static int paged_decode_impl(const void *q, int64_t q_batch_stride, int64_t q_he
                              int64_t gate_batch_stride, int64_t gate_head_stride, void *stream,
                              const void *k_new = nullptr, int64_t k_new_row_stride = 0, const void *v_new = nullptr,
                              int64_t v_new_row_stride = 0, const int32_t *slot_mapping = nullptr,
-                             int new_dtype = -1) {
+                             int new_dtype = -1, void *counters = nullptr) {
   if (batch == 0) return NQ_OK;
   if (batch < 0 || batch > 65535 || num_q_heads <= 0 || num_kv_heads <= 0 || num_kv_heads > 65535)
     return fail(NQ_EINVAL, "paged_decode: bad batch/head counts");
@@ -1178,6 +1349,7 @@ static int paged_decode_impl(const void *q, int64_t q_batch_stride, int64_t q_he
     a.ws_o = static_cast<float *>(workspace);
     a.ws_lse = reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + (n * head_dim * 4 + 255) / 256 * 256);
   }
+  a.counters = static_cast<unsigned *>(counters);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (q_dtype == NQ_BF16)
     return head_dim == 256
@@ -1241,6 +1413,79 @@ extern "C" int nq_paged_decode_store(const void *q, int64_t q_batch_stride, int6
                            v_new, v_new_row_stride, slot_mapping, new_dtype);
 }
 
+// Whether a decode of these sizes runs as one launch (paged_decode_fused_kernel),
+// and its splits: about one workgroup per CU at the longest contexts the table
+// allows, of 128 to 512 tokens, and at most 32 splits per sequence.  A chain of
+// memory round trips decides at these sizes; the merge inside the launch costs
+// three of them (the partials' completion, the count, the loads) against a
+// second launch's 4 us.  Measured, a captured step of 8 layers, two launches ->
+// one: head_dim 256, 6 rows of 150-3000 tokens 274 -> 220 us, 16 rows of
+// 500-2000 276 -> 236, fp8 271 -> 196 (their stream-K merge and one-step prefetch
+// are the slower side); fp8 at 128, 4 rows of 1000-2000 tokens 240 -> 174, 16 of
+// 1000-4000 326 -> 319; 16-bit at 128, one row of 700 tokens 189 -> 168, two of
+// 2000 with 2 kv heads 153 -> 144, but one of 4000 with 8 204 -> 207, 8 of
+// 300-2000 208 -> 228: there only up to kFusedTokens tokens x kv heads, and for
+// tables of at most 512 tokens (32 rows of 100-500: 219 -> 199).
+constexpr int64_t kFusedTokens = 16384;
+static bool decode_fused_plan(int batch, int num_kv_heads, int head_dim, int64_t max_tokens, int block_size, bool fp8,
+                              int *num_splits, int *split_tokens) {
+  // an explicit choice of splits or schedule is one of the two-launch path's
+  if (getenv("NQ_DECODE_SPLIT_TOKENS") || getenv("NQ_DECODE_STREAMK")) return false;
+  const int64_t tokens = static_cast<int64_t>(batch) * num_kv_heads * max_tokens;
+  const int64_t cus = device_cus();
+  const bool short_table = max_tokens <= 512;
+  if (head_dim == 128 && !fp8 && tokens > kFusedTokens && !short_table) return false;
+  int64_t split = std::max((tokens + cus - 1) / cus, (max_tokens + 31) / 32);
+  split = std::max<int64_t>(128, (split + 127) / 128 * 128);
+  if (short_table && static_cast<int64_t>(batch) * num_kv_heads <= 4 * cus) split = std::min<int64_t>(split, 512);
+  if (split > 512 || split > max_split_tokens(block_size)) return false;
+  *num_splits = static_cast<int>((max_tokens + split - 1) / split);
+  *split_tokens = static_cast<int>(split);
+  return true;
+}
+
+extern "C" int nq_decode_config(int batch, int num_q_heads, int num_kv_heads, int head_dim, int max_blocks_per_seq,
+                                int block_size, int kv_dtype, int64_t *config) {
+  if (!config || batch <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0 || max_blocks_per_seq <= 0 ||
+      block_size <= 0)
+    return fail(NQ_EINVAL, "decode_config: bad arguments");
+  int ns = 0, st = 0;
+  const int64_t max_tokens = static_cast<int64_t>(max_blocks_per_seq) * block_size;
+  const bool fused = decode_fused_plan(batch, num_kv_heads, head_dim, max_tokens, block_size, kv_dtype == NQ_FP8_E4M3, &ns, &st);
+  if (!fused) {
+    const int rc =
+        nq_decode_plan(batch, num_q_heads, num_kv_heads, max_blocks_per_seq, block_size, kv_dtype, &ns, &st);
+    if (rc != NQ_OK) return rc;
+  }
+  config[0] = fused ? static_cast<int64_t>(batch) * num_kv_heads * kCounterBytes : 0;
+  config[1] = ns;
+  config[2] = st;
+  config[3] = nq_decode_workspace_bytes(batch, num_q_heads, head_dim, ns);
+  return NQ_OK;
+}
+
+extern "C" int nq_paged_decode_fused(const void *q, int64_t q_batch_stride, int64_t q_head_stride,
+                                     void *k_cache, void *v_cache, const int32_t *block_tables, int64_t bt_stride,
+                                     int max_blocks_per_seq, const int32_t *context_lens, const void *k_new,
+                                     int64_t k_new_row_stride, const void *v_new, int64_t v_new_row_stride,
+                                     const int32_t *slot_mapping, int new_dtype, void *out,
+                                     int64_t out_batch_stride, int64_t out_head_stride, int batch,
+                                     int num_q_heads, int num_kv_heads, int head_dim, int block_size,
+                                     int64_t num_blocks, float softmax_scale, int num_splits, int split_tokens,
+                                     void *workspace, int64_t workspace_bytes, int q_dtype, int kv_dtype,
+                                     const float *k_scale, const float *v_scale, const void *gate,
+                                     int64_t gate_batch_stride, int64_t gate_head_stride, void *counters,
+                                     int64_t counter_bytes, void *stream) {
+  if (!counters || counter_bytes < static_cast<int64_t>(batch) * num_kv_heads * kCounterBytes || !aligned(counters, 64))
+    return fail(NQ_EINVAL, "paged_decode_fused: %lld bytes of counters at %p", (long long)counter_bytes, counters);
+  return paged_decode_impl(q, q_batch_stride, q_head_stride, k_cache, v_cache, block_tables, bt_stride,
+                           max_blocks_per_seq, context_lens, out, out_batch_stride, out_head_stride, batch,
+                           num_q_heads, num_kv_heads, head_dim, block_size, num_blocks, softmax_scale,
+                           num_splits, split_tokens, workspace, workspace_bytes, q_dtype, kv_dtype, k_scale,
+                           v_scale, gate, gate_batch_stride, gate_head_stride, stream, k_new, k_new_row_stride,
+                           v_new, v_new_row_stride, slot_mapping, new_dtype, counters);
+}
+
 // ---------------------------------------------------------------------------
 // nq_paged_decode_noalloc: the same kernels with the split-K partials in a
 // static device array, for callers that cannot allocate.  Every call on a
@@ -1250,6 +1495,10 @@ extern "C" int nq_paged_decode_store(const void *q, int64_t q_batch_stride, int6
 namespace {
 constexpr int64_t kScratchBytes = NQ_DECODE_NOALLOC_SCRATCH_BYTES;  // per device
 constexpr int kMaxDevices = 64;
+__global__ __launch_bounds__(256) void zero_words_kernel(unsigned *p, int n) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) p[i] = 0u;
+}
 __device__ __attribute__((aligned(256))) uint8_t scratch[kScratchBytes];
 std::mutex g_scratch_mu;
 void *g_scratch_ptr[kMaxDevices];
@@ -1288,6 +1537,29 @@ extern "C" int nq_paged_decode_noalloc(const void *q, int64_t q_batch_stride, in
   void *ws = nullptr;
   const int rc = scratch_address(&ws);
   if (rc != NQ_OK) return rc;
+  // A small batch takes the kernel that nq_decode_config gives it, with that
+  // plan, so that results do not depend on where the partials live.  Its
+  // counters are the array's first bytes, zeroed ahead of each launch: unlike a
+  // caller's they must not carry anything from calls that raced.
+  int fs = 0, ft = 0;
+  const int64_t max_tokens = static_cast<int64_t>(max_blocks_per_seq) * block_size;
+  if (batch > 0 && batch <= 65535 && num_kv_heads > 0 && max_tokens > 0 && num_splits > 0 && split_tokens > 0 &&
+      split_tokens % 128 == 0 && num_splits * static_cast<int64_t>(split_tokens) >= max_tokens &&
+      decode_fused_plan(batch, num_kv_heads, head_dim, max_tokens, block_size, kv_dtype == NQ_FP8_E4M3, &fs, &ft)) {
+    const int64_t cb = (static_cast<int64_t>(batch) * num_kv_heads * kCounterBytes + 255) / 256 * 256;
+    if (cb + nq_decode_workspace_bytes(batch, num_q_heads, head_dim, fs) <= kScratchBytes) {
+      hipStream_t s = static_cast<hipStream_t>(stream);
+      const int words = static_cast<int>(cb / 4);
+      zero_words_kernel<<<(words + 255) / 256, 256, 0, s>>>(static_cast<unsigned *>(ws), words);
+      const int zrc = check_launch("paged_decode_noalloc(counters)");
+      if (zrc != NQ_OK) return zrc;
+      return paged_decode_impl(q, q_batch_stride, q_head_stride, k_cache, v_cache, block_tables, bt_stride,
+                               max_blocks_per_seq, context_lens, out, out_batch_stride, out_head_stride, batch,
+                               num_q_heads, num_kv_heads, head_dim, block_size, num_blocks, softmax_scale, fs, ft,
+                               static_cast<uint8_t *>(ws) + cb, kScratchBytes - cb, q_dtype, kv_dtype, k_scale,
+                               v_scale, nullptr, 0, 0, stream, nullptr, 0, nullptr, 0, nullptr, -1, ws);
+    }
+  }
   if (num_splits > 1) {
     int64_t need = nq_decode_workspace_bytes(batch, num_q_heads, head_dim, num_splits);
     if (need > kScratchBytes && split_tokens > 0 && max_blocks_per_seq > 0) {

@@ -15,11 +15,12 @@ from __future__ import annotations
 
 import ctypes
 import os
+import threading
 
 import torch
 
 from . import _lib
-from ._lib import check, dtype_code, lib, ptr, require_cuda, stream_of
+from ._lib import check, dtype_code, lib, ptr, require_cuda, stream_of  # noqa: F401
 
 # Persistent device buffers of the kernels, one per (device, stream): calls
 # on one stream are ordered, so they may share a buffer; calls on different
@@ -34,6 +35,12 @@ _prefill_queues: dict[tuple[int, int], torch.Tensor] = {}
 _prefill_parts: dict[tuple[int, int], torch.Tensor] = {}
 _gdn_segments: dict[tuple[int, int], torch.Tensor] = {}
 _retired: list[torch.Tensor] = []
+# Zeroed arrival counters of the one-launch decode: a pool per device, a slot
+# per (device, stream).
+_COUNTER_SLOTS, _COUNTER_SLOT_BYTES = 32, 128 << 10
+_counter_pools: dict[int, torch.Tensor] = {}
+_decode_counters: dict[tuple[int, int], torch.Tensor] = {}
+_counter_lock = threading.Lock()
 _DEBUG_QUEUE = os.environ.get("NQ_DEBUG_PREFILL_QUEUE", "0") not in ("", "0")
 
 
@@ -69,10 +76,12 @@ def release_workspaces(device=None) -> int:
     at zero again)."""
     idx = None if device is None else _key(device)[0]
     n = 0
-    for table in (_workspaces, _prefill_queues, _prefill_parts, _gdn_segments):
+    for table in (_workspaces, _prefill_queues, _prefill_parts, _gdn_segments, _decode_counters):
         for key in [k for k in table if idx is None or k[0] == idx]:
             del table[key]
             n += 1
+    for dev in [k for k in _counter_pools if idx is None or k == idx]:
+        del _counter_pools[dev]
     keep = [t for t in _retired if idx is not None and t.device.index != idx]
     n += len(_retired) - len(keep)
     _retired[:] = keep
@@ -149,9 +158,38 @@ def reserve_decode_workspace(device, max_batch, num_q_heads, num_kv_heads, max_b
     for b in range(1, int(max_batch) + 1):
         ns, _ = decode_plan(b, num_q_heads, num_kv_heads, max_blocks_per_seq, block_size, kv_dtype)
         need = max(need, lib().nq_decode_workspace_bytes(b, num_q_heads, head_dim, ns))
+        config = (ctypes.c_int64 * 4)()    # the one-launch path's own plan
+        check(lib().nq_decode_config(b, num_q_heads, num_kv_heads, head_dim, max_blocks_per_seq, block_size,
+                                     dtype_code(kv_dtype), config), "decode_config")
+        need = max(need, config[3])
     if need > 0:
         decode_workspace(device, need)
     return need
+
+
+def _decode_counter_slot(device, nbytes: int) -> torch.Tensor | None:
+    """Arrival counters of the one-launch decode for the current stream of
+    ``device``: a slot of the device's pool, which is zeroed and waited for
+    when it is made (every launch leaves its counters zero again), so that a
+    stream that is being captured can take one.  ``None`` -- the caller then
+    takes the two-launch path -- when the pool would have to be made during a
+    capture, has no slot left or too small ones."""
+    key = _key(device)
+    slot = _decode_counters.get(key)
+    if slot is None:
+        pool = _counter_pools.get(key[0])
+        if pool is None:
+            if torch.cuda.is_current_stream_capturing():
+                return None
+            pool = torch.zeros(_COUNTER_SLOTS, _COUNTER_SLOT_BYTES // 4, dtype=torch.int32, device=device)
+            torch.cuda.current_stream(key[0]).synchronize()
+            _counter_pools[key[0]] = pool
+        with _counter_lock:
+            used = sum(k[0] == key[0] for k in _decode_counters)
+            if used >= _COUNTER_SLOTS:
+                return None
+            slot = _decode_counters.setdefault(key, pool[used])
+    return slot if nbytes <= _COUNTER_SLOT_BYTES else None
 
 
 def prefill_workspace(device) -> torch.Tensor:
@@ -216,8 +254,15 @@ def paged_decode(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale,
         out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     o3 = out.squeeze(1) if out.dim() == 4 else out
     W = block_table.shape[1]
-    ns, st = decode_plan(B, hq, hkv, W, bs, k_cache.dtype)
-    wsb = lib().nq_decode_workspace_bytes(B, hq, d, ns)
+    config = (ctypes.c_int64 * 4)()
+    check(lib().nq_decode_config(B, hq, hkv, d, W, bs, dtype_code(k_cache.dtype), config), "decode_config")
+    counter_bytes, ns, st, wsb = config
+    counters = None
+    if counter_bytes > 0:    # a small batch: one launch
+        counters = _decode_counter_slot(q.device, counter_bytes)
+        if counters is None:
+            ns, st = decode_plan(B, hq, hkv, W, bs, k_cache.dtype)
+            wsb = lib().nq_decode_workspace_bytes(B, hq, d, ns)
     ws = decode_workspace(q.device, wsb)
     args = (ptr(q3), q3.stride(0), q3.stride(1), ptr(k_cache), ptr(v_cache), ptr(block_table),
             block_table.stride(0), W, ptr(cache_seqlens), ptr(o3), o3.stride(0), o3.stride(1),
@@ -241,6 +286,19 @@ def paged_decode(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale,
             raise RuntimeError("paged_decode: k/v dtype must match the cache (or be stored into an fp8 cache)")
         if slot_mapping.dtype != torch.int32 or slot_mapping.numel() != B:
             raise RuntimeError("paged_decode: slot_mapping must be int32 [B]")
+    if counters is not None:
+        new = k is not None
+        rc = lib().nq_paged_decode_fused(
+            ptr(q3), q3.stride(0), q3.stride(1), ptr(k_cache), ptr(v_cache), ptr(block_table),
+            block_table.stride(0), W, ptr(cache_seqlens), ptr(k3) if new else None, k3.stride(0) if new else 0,
+            ptr(v3) if new else None, v3.stride(0) if new else 0, ptr(slot_mapping) if new else None,
+            dtype_code(k3.dtype) if new else -1, ptr(o3), o3.stride(0), o3.stride(1),
+            B, hq, hkv, d, bs, nb, float(softmax_scale), ns, st, ptr(ws), 0 if ws is None else ws.numel(),
+            dtype_code(q.dtype), dtype_code(k_cache.dtype), ptr(k_scale) if fp8 else None,
+            ptr(v_scale) if fp8 else None, ptr(g3) if g3 is not None else None,
+            0 if g3 is None else g3.stride(0), 0 if g3 is None else g3.stride(1), ptr(counters),
+            counters.numel() * 4, stream_of(q))
+    elif k is not None:
         rc = lib().nq_paged_decode_store(
             ptr(q3), q3.stride(0), q3.stride(1), ptr(k_cache), ptr(v_cache), ptr(block_table),
             block_table.stride(0), W, ptr(cache_seqlens), ptr(k3), k3.stride(0), ptr(v3), v3.stride(0),
