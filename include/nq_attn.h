@@ -390,6 +390,20 @@ int nq_prepare_decode(const int64_t *sampled_token_ids, const int64_t *batch_slo
                       int num_seqs, int block_size, void *stream);
 
 /*
+ * The static inputs of a captured decode step from a batch's own tensors, in
+ * one launch (engine/model_runner.py:325-334, there one copy or fill each):
+ * rows i < batch of input_ids, positions, slot_mapping, context_lens and
+ * block_tables [batch, width] are copied; rows batch .. rows - 1 get
+ * to_slot_mapping -1 and to_context_lens 0.  The int64 and int32 vectors are
+ * contiguous; table row strides in elements.
+ */
+int nq_stage_decode(const int64_t *input_ids, const int64_t *positions, const int32_t *slot_mapping,
+                    const int32_t *context_lens, const int32_t *block_tables, int64_t bt_stride,
+                    int batch, int width, int64_t *to_input_ids, int64_t *to_positions,
+                    int32_t *to_slot_mapping, int32_t *to_context_lens, int32_t *to_block_tables,
+                    int64_t to_bt_stride, int rows, void *stream);
+
+/*
  * Fused q/k Gemma RMS norm + partial rotary embedding + KV-cache store.
  * Replaces, in Qwen3_5Attention.forward (models/qwen3_5.py:135-137), the
  * calls q_norm(query), k_norm(key) (GemmaRMSNorm, layers/layernorm.py:81-91)

@@ -268,13 +268,16 @@ class ModelRunner:
         context = get_context()
         graph = self.graphs[next(x for x in self.graph_bs if x >= bs)]
         gv = self.graph_vars
-        gv["input_ids"][:bs] = input_ids
-        gv["positions"][:bs] = positions
-        gv["slot_mapping"].fill_(-1)
-        gv["slot_mapping"][:bs] = context.slot_mapping
-        gv["context_lens"].zero_()
-        gv["context_lens"][:bs] = context.context_lens
-        gv["block_tables"][:bs, :context.block_tables.size(1)] = context.block_tables
+        if not kernels.stage_decode(input_ids, positions, context.slot_mapping, context.context_lens,
+                                    context.block_tables, gv["input_ids"], gv["positions"], gv["slot_mapping"],
+                                    gv["context_lens"], gv["block_tables"]):
+            gv["input_ids"][:bs] = input_ids
+            gv["positions"][:bs] = positions
+            gv["slot_mapping"].fill_(-1)
+            gv["slot_mapping"][:bs] = context.slot_mapping
+            gv["context_lens"].zero_()
+            gv["context_lens"][:bs] = context.context_lens
+            gv["block_tables"][:bs, :context.block_tables.size(1)] = context.block_tables
         graph.replay()
         return self._logits(gv["outputs"][:bs])
 

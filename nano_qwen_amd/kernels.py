@@ -401,6 +401,33 @@ def prepare_decode(sampled_token_ids, batch_slots, seq_lens, last_block_ids, inp
     check(rc, "prepare_decode")
 
 
+def stage_decode(input_ids, positions, slot_mapping, context_lens, block_tables, to_input_ids, to_positions,
+                 to_slot_mapping, to_context_lens, to_block_tables) -> bool:
+    """A decode batch's inputs into the static inputs of a captured step, in
+    one launch; rows past the batch become padding (slot -1, context 0).
+    Returns False, with nothing done, for tensors that do not lie on one device
+    in the types and layouts ``prepare_decode`` leaves."""
+    n, rows = input_ids.shape[0], to_input_ids.shape[0]
+    dev = to_input_ids.device
+    for t, to, dtype in ((input_ids, to_input_ids, torch.int64), (positions, to_positions, torch.int64),
+                         (slot_mapping, to_slot_mapping, torch.int32), (context_lens, to_context_lens, torch.int32)):
+        if t.shape != (n,) or to.shape != (rows,) or t.dtype != dtype or to.dtype != dtype or t.device != dev \
+                or to.device != dev or (n > 1 and t.stride(0) != 1) or (rows > 1 and to.stride(0) != 1):
+            return False
+    b, tb = block_tables, to_block_tables
+    if b.dim() != 2 or tb.dim() != 2 or b.shape[0] != n or tb.shape[0] < n or b.shape[1] > tb.shape[1] \
+            or b.dtype != torch.int32 or tb.dtype != torch.int32 or b.device != dev or tb.device != dev \
+            or dev.type != "cuda" or rows < n or (b.shape[1] > 1 and b.stride(1) != 1) \
+            or tb.stride(1) != 1 or tb.stride(0) < b.shape[1]:
+        return False
+    rc = lib().nq_stage_decode(ptr(input_ids), ptr(positions), ptr(slot_mapping), ptr(context_lens), ptr(b),
+                               b.stride(0), n, b.shape[1], ptr(to_input_ids), ptr(to_positions),
+                               ptr(to_slot_mapping), ptr(to_context_lens), ptr(tb), tb.stride(0), rows,
+                               stream_of(to_input_ids))
+    check(rc, "stage_decode")
+    return True
+
+
 def qk_norm_rope_store(positions, query, key, value, q_weight, k_weight, eps, cos_sin_cache, rotary_dim,
                        k_cache=None, v_cache=None, slot_mapping=None, k_scale=None, v_scale=None,
                        weight_offset=1.0, q_out=None, k_out=None, _return_args=False):

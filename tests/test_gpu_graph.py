@@ -131,3 +131,31 @@ def test_decode_graph_buckets(cuda, kv_dtype):
         assert_close(out_g.view(bs, HQ, D).float().cpu().numpy(), ref.cpu().numpy(), what=f"graph bs={bs}",
                      max_abs=L * tol["max_abs"], mean_abs=L * tol["mean_abs"])
 
+
+
+@pytest.mark.parametrize("n,rows,w,width", [(1, 1, 1, 1), (3, 8, 5, 12), (8, 8, 12, 12), (300, 512, 129, 130), (0, 4, 1, 3)])
+def test_stage_decode(cuda, n, rows, w, width):
+    """One launch leaves the static inputs as the copies and fills do; tensors of
+    another type, layout or width are left to those."""
+    from nano_qwen_amd import kernels
+    g = torch.Generator().manual_seed(n)
+    ints = lambda dtype, *shape: torch.randint(-5, 1 << 30, shape, generator=g, dtype=dtype).to(cuda)
+    src = [ints(torch.int64, n), ints(torch.int64, n), ints(torch.int32, n), ints(torch.int32, n),
+           ints(torch.int32, n, w + 3)[:, :w]]
+    dst = [ints(torch.int64, rows), ints(torch.int64, rows), ints(torch.int32, rows), ints(torch.int32, rows),
+           ints(torch.int32, rows, width)]
+    want = [t.clone() for t in dst]
+    want[2].fill_(-1)
+    want[3].zero_()
+    for i in range(4):
+        want[i][:n] = src[i]
+    want[4][:n, :w] = src[4]
+    assert kernels.stage_decode(*src, *dst)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(dst, want))
+    for i, bad in ((0, src[0].int()), (2, src[2].repeat(2)[::2] if n > 1 else src[2].long()), (3, src[3].cpu()),
+                   (4, ints(torch.int32, n, width + 1))):
+        before = [t.clone() for t in dst]
+        assert not kernels.stage_decode(*src[:i], bad, *src[i + 1:], *dst)
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(dst, before))
