@@ -225,6 +225,23 @@ int nq_paged_decode_fused(const void *q, int64_t q_batch_stride, int64_t q_head_
                           int64_t gate_batch_stride, int64_t gate_head_stride, void *counters,
                           int64_t counter_bytes, void *stream);
 
+/* The two above in one call: the plan that nq_decode_config gives (that of
+ * nq_decode_plan without enough counters) and its launch; k_new and gate are
+ * optional.  Returns 1, with nothing launched and the bytes in *need, when the
+ * plan needs a larger workspace. */
+int nq_paged_decode_auto(const void *q, int64_t q_batch_stride, int64_t q_head_stride,
+                         void *k_cache, void *v_cache, const int32_t *block_tables, int64_t bt_stride,
+                         int max_blocks_per_seq, const int32_t *context_lens, const void *k_new,
+                         int64_t k_new_row_stride, const void *v_new, int64_t v_new_row_stride,
+                         const int32_t *slot_mapping, int new_dtype, void *out,
+                         int64_t out_batch_stride, int64_t out_head_stride, int batch,
+                         int num_q_heads, int num_kv_heads, int head_dim, int block_size,
+                         int64_t num_blocks, float softmax_scale, void *workspace,
+                         int64_t workspace_bytes, int q_dtype, int kv_dtype, const float *k_scale,
+                         const float *v_scale, const void *gate, int64_t gate_batch_stride,
+                         int64_t gate_head_stride, void *counters, int64_t counter_bytes, int64_t *need,
+                         void *stream);
+
 /* How a decode of these sizes runs best, in config[4]: bytes of counters of
  * nq_paged_decode_fused (0: nq_paged_decode or nq_paged_decode_store instead),
  * num_splits, split_tokens, bytes of workspace.  Host-known sizes only. */
@@ -343,9 +360,10 @@ int nq_varlen_prefill_gated(const void *q, int64_t q_row_stride, int64_t q_head_
  * short prompt, a few new tokens behind long prefixes): each queue's key tiles
  * are cut into one equal range per workgroup, and a second kernel merges the
  * float32 partial outputs of the items that a cut crosses.  Launches with
- * enough items, or whose split_workspace is null or smaller than
- * nq_prefill_split_workspace_bytes, run as the two calls above; gate may be
- * null.  total_q: rows of q (the items are bounded from it).  split_workspace
+ * enough items run as the two calls above, and so do those whose
+ * split_workspace is null or smaller than nq_prefill_split_workspace_bytes,
+ * unless need is given: then nothing is launched, *need is set to those bytes
+ * and 1 returned.  gate may be null.  total_q: rows of q (the items are bounded from it).  split_workspace
  * must be 256-byte aligned; its contents need no clearing.  Calls that overlap
  * may not share one.
  */
@@ -363,7 +381,7 @@ int nq_varlen_prefill_split(const void *q, int64_t q_row_stride, int64_t q_head_
                             void *workspace, int64_t workspace_bytes,
                             const void *gate, int64_t gate_row_stride, int64_t gate_head_stride,
                             int64_t total_q, void *split_workspace, int64_t split_workspace_bytes,
-                            void *stream);
+                            int64_t *need, void *stream);
 
 /* Bytes of split_workspace with which nq_varlen_prefill_split cuts a launch of
  * these sizes into equal ranges; 0: it would not (decided from the sizes and
@@ -518,8 +536,10 @@ int nq_gdn_prefill(const void *q, int64_t q_row_stride, const void *k, int64_t k
  * each sequence is cut into segments that run side by side, once for their
  * states and once, after a float32 chaining of those, for the outputs (same
  * results up to the order of float32 sums).  total_tokens: rows of q.  A null
- * or smaller workspace than nq_gdn_prefill_workspace_bytes, or a launch for
- * which that is 0, runs as nq_gdn_prefill.  workspace must be 256-byte
+ * or smaller workspace than nq_gdn_prefill_workspace_bytes runs as
+ * nq_gdn_prefill, unless need is given: then nothing is launched, *need is set to
+ * those bytes and 1 returned.  A launch for which they are 0 runs as
+ * nq_gdn_prefill.  workspace must be 256-byte
  * aligned; its contents need no clearing.  Calls that overlap may not share
  * one.
  */
@@ -530,7 +550,7 @@ int nq_gdn_prefill_split(const void *q, int64_t q_row_stride, const void *k, int
                          const int32_t *state_indices, int64_t num_slots, int initial_state_from_slot,
                          void *out, int64_t out_row_stride, int num_k_heads, int num_v_heads,
                          int head_k_dim, int head_v_dim, int dtype, int64_t total_tokens,
-                         void *workspace, int64_t workspace_bytes, void *stream);
+                         void *workspace, int64_t workspace_bytes, int64_t *need, void *stream);
 
 /* Bytes of workspace with which nq_gdn_prefill_split cuts a launch of these
  * sizes into segments; 0: it would not (decided from the sizes and the current

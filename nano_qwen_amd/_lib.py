@@ -57,6 +57,11 @@ _SIGS = {
                                   c_int64, c_int64, c_int, c_int, c_int, c_int, c_int, c_float, c_int,
                                   c_int, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
     "nq_decode_config": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int, POINTER(c_int64)]),
+    "nq_paged_decode_auto": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_int,
+                                     c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int, c_void_p,
+                                     c_int64, c_int64, c_int, c_int, c_int, c_int, c_int, c_int64, c_float,
+                                     c_void_p, c_int64, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int64,
+                                     c_int64, c_void_p, c_int64, POINTER(c_int64), c_void_p]),
     "nq_paged_decode_fused": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_int,
                                       c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int, c_void_p,
                                       c_int64, c_int64, c_int, c_int, c_int, c_int, c_int, c_int64, c_float, c_int,
@@ -72,7 +77,7 @@ _SIGS = {
                                         c_void_p, c_int, c_int, c_void_p, c_int64, c_int, c_int64, c_void_p,
                                         c_int64, c_int64, c_int, c_int, c_int, c_int, c_int, c_float, c_int,
                                         c_int, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64,
-                                        c_int64, c_int64, c_void_p, c_int64, c_void_p]),
+                                        c_int64, c_int64, c_void_p, c_int64, POINTER(c_int64), c_void_p]),
     "nq_prefill_split_workspace_bytes": (c_int64, [c_int, c_int64, c_int, c_int, c_int, c_int, c_int]),
     "nq_prepare_decode": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                   c_void_p, c_int, c_int, c_void_p]),
@@ -87,7 +92,7 @@ _SIGS = {
     "nq_gdn_prefill_split": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64,
                                      c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                                      c_int64, c_int, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int, c_int64,
-                                     c_void_p, c_int64, c_void_p]),
+                                     c_void_p, c_int64, POINTER(c_int64), c_void_p]),
     "nq_gdn_prefill_workspace_bytes": (c_int64, [c_int, c_int64, c_int]),
     "nq_gated_rmsnorm": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_float, c_void_p, c_int64,
                                  c_int64, c_int, c_int, c_void_p]),
@@ -138,11 +143,22 @@ def dtype_code(t: torch.dtype) -> int:
 
 
 def ptr(t):
-    return None if t is None else c_void_p(t.data_ptr())
+    """A tensor's address (an int, which a void pointer argument takes as it is)."""
+    return None if t is None else t.data_ptr()
 
 
-def stream_of(t: torch.Tensor) -> c_void_p:
-    return c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+def raw_stream(index: int) -> int:
+    """The current stream's handle on device ``index``."""
+    return torch.cuda.current_stream(index).cuda_stream
+
+
+# The same from torch's C side where it exists (a stream object costs about
+# 2 us of the 25-30 of a small launch).
+raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", raw_stream)
+
+
+def stream_of(t: torch.Tensor) -> int:
+    return raw_stream(t.get_device())
 
 
 def require_cuda(*tensors, what: str) -> None:

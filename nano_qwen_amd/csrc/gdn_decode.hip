@@ -332,13 +332,22 @@ extern "C" int nq_gdn_prefill(const void *q, int64_t q_row_stride, const void *k
                           stream);
 }
 
+extern "C" int64_t nq_gdn_prefill_workspace_bytes(int num_seqs, int64_t total_tokens, int num_v_heads);
+
 extern "C" int nq_gdn_prefill_split(const void *q, int64_t q_row_stride, const void *k, int64_t k_row_stride,
                               const void *v, int64_t v_row_stride, const void *a, int64_t a_row_stride,
                               const void *b, int64_t b_row_stride, const float *A_log, const float *dt_bias,
                               const int32_t *cu_seqlens, int num_seqs, float *state, const int32_t *state_indices,
                               int64_t num_slots, int initial_state_from_slot, void *out, int64_t out_row_stride,
                               int num_k_heads, int num_v_heads, int head_k_dim, int head_v_dim, int dtype,
-                              int64_t total_tokens, void *workspace, int64_t workspace_bytes, void *stream) {
+                              int64_t total_tokens, void *workspace, int64_t workspace_bytes, int64_t *need, void *stream) {
+  if (need) {
+    const int64_t bytes = nq_gdn_prefill_workspace_bytes(num_seqs, total_tokens, num_v_heads);
+    if (bytes > 0 && (!workspace || workspace_bytes < bytes)) {
+      *need = bytes;
+      return 1;
+    }
+  }
   return gdn_prefill_impl(q, q_row_stride, k, k_row_stride, v, v_row_stride, a, a_row_stride, b, b_row_stride, A_log,
                           dt_bias, cu_seqlens, num_seqs, state, state_indices, num_slots, initial_state_from_slot, out,
                           out_row_stride, num_k_heads, num_v_heads, head_k_dim, head_v_dim, dtype, total_tokens,

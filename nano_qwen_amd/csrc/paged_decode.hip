@@ -1492,6 +1492,42 @@ extern "C" int nq_paged_decode_fused(const void *q, int64_t q_batch_stride, int6
                            v_new, v_new_row_stride, slot_mapping, new_dtype, counters);
 }
 
+extern "C" int nq_paged_decode_auto(const void *q, int64_t q_batch_stride, int64_t q_head_stride,
+                                    void *k_cache, void *v_cache, const int32_t *block_tables, int64_t bt_stride,
+                                    int max_blocks_per_seq, const int32_t *context_lens, const void *k_new,
+                                    int64_t k_new_row_stride, const void *v_new, int64_t v_new_row_stride,
+                                    const int32_t *slot_mapping, int new_dtype, void *out,
+                                    int64_t out_batch_stride, int64_t out_head_stride, int batch,
+                                    int num_q_heads, int num_kv_heads, int head_dim, int block_size,
+                                    int64_t num_blocks, float softmax_scale, void *workspace,
+                                    int64_t workspace_bytes, int q_dtype, int kv_dtype, const float *k_scale,
+                                    const float *v_scale, const void *gate, int64_t gate_batch_stride,
+                                    int64_t gate_head_stride, void *counters, int64_t counter_bytes, int64_t *need,
+                                    void *stream) {
+  int64_t config[4];
+  int rc = nq_decode_config(batch, num_q_heads, num_kv_heads, head_dim, max_blocks_per_seq, block_size, kv_dtype, config);
+  if (rc != NQ_OK) return rc;
+  const bool fused = config[0] > 0 && counters && counter_bytes >= config[0];
+  int ns = static_cast<int>(config[1]), st = static_cast<int>(config[2]);
+  int64_t bytes = config[3];
+  if (config[0] > 0 && !fused) {  // no counters: two launches
+    rc = nq_decode_plan(batch, num_q_heads, num_kv_heads, max_blocks_per_seq, block_size, kv_dtype, &ns, &st);
+    if (rc != NQ_OK) return rc;
+    bytes = nq_decode_workspace_bytes(batch, num_q_heads, head_dim, ns);
+  }
+  if (bytes > 0 && (!workspace || workspace_bytes < bytes)) {
+    if (!need) return fail(NQ_EINVAL, "paged_decode_auto: workspace %lld bytes < %lld", (long long)workspace_bytes, (long long)bytes);
+    *need = bytes;
+    return 1;
+  }
+  return paged_decode_impl(q, q_batch_stride, q_head_stride, k_cache, v_cache, block_tables, bt_stride,
+                           max_blocks_per_seq, context_lens, out, out_batch_stride, out_head_stride, batch,
+                           num_q_heads, num_kv_heads, head_dim, block_size, num_blocks, softmax_scale,
+                           ns, st, workspace, workspace_bytes, q_dtype, kv_dtype, k_scale,
+                           v_scale, gate, gate_batch_stride, gate_head_stride, stream, k_new, k_new_row_stride,
+                           v_new, v_new_row_stride, slot_mapping, new_dtype, fused ? counters : nullptr);
+}
+
 // ---------------------------------------------------------------------------
 // nq_paged_decode_noalloc: the same kernels with the split-K partials in a
 // static device array, for callers that cannot allocate.  Every call on a

@@ -1874,7 +1874,16 @@ extern "C" int nq_varlen_prefill_split(
     void *out, int64_t out_row_stride, int64_t out_head_stride, int num_seqs, int num_q_heads, int num_kv_heads,
     int head_dim, int block_size, float softmax_scale, int causal, int q_dtype, int kv_dtype, const float *k_scale,
     const float *v_scale, void *workspace, int64_t workspace_bytes, const void *gate, int64_t gate_row_stride,
-    int64_t gate_head_stride, int64_t total_q, void *split_workspace, int64_t split_workspace_bytes, void *stream) {
+    int64_t gate_head_stride, int64_t total_q, void *split_workspace, int64_t split_workspace_bytes, int64_t *need,
+    void *stream) {
+  if (need) {
+    const int64_t bytes = nq_prefill_split_workspace_bytes(num_seqs, total_q, max_seqlen_q, max_seqlen_k, num_q_heads,
+                                                           num_kv_heads, head_dim);
+    if (bytes > 0 && (!split_workspace || split_workspace_bytes < bytes)) {
+      *need = bytes;
+      return 1;
+    }
+  }
   return varlen_prefill_impl(q, q_row_stride, q_head_stride, k, v, kv_row_stride, cu_seqlens_q, cu_seqlens_k,
                              max_seqlen_q, max_seqlen_k, block_tables, bt_stride, max_blocks_per_seq, num_blocks,
                              out, out_row_stride, out_head_stride, num_seqs, num_q_heads, num_kv_heads, head_dim,

@@ -20,7 +20,7 @@ import threading
 import torch
 
 from . import _lib
-from ._lib import check, dtype_code, lib, ptr, require_cuda, stream_of  # noqa: F401
+from ._lib import check, dtype_code, lib, ptr, raw_stream, require_cuda, stream_of
 
 # Persistent device buffers of the kernels, one per (device, stream): calls
 # on one stream are ordered, so they may share a buffer; calls on different
@@ -47,7 +47,7 @@ _DEBUG_QUEUE = os.environ.get("NQ_DEBUG_PREFILL_QUEUE", "0") not in ("", "0")
 def _key(device) -> tuple[int, int]:
     dev = torch.device(device)
     idx = dev.index if dev.index is not None else torch.cuda.current_device()
-    return idx, torch.cuda.current_stream(idx).cuda_stream
+    return idx, raw_stream(idx)
 
 
 def _grow(table, key, nbytes, dtype, device, zero=False):
@@ -167,29 +167,29 @@ def reserve_decode_workspace(device, max_batch, num_q_heads, num_kv_heads, max_b
     return need
 
 
-def _decode_counter_slot(device, nbytes: int) -> torch.Tensor | None:
-    """Arrival counters of the one-launch decode for the current stream of
-    ``device``: a slot of the device's pool, which is zeroed and waited for
-    when it is made (every launch leaves its counters zero again), so that a
-    stream that is being captured can take one.  ``None`` -- the caller then
-    takes the two-launch path -- when the pool would have to be made during a
-    capture, has no slot left or too small ones."""
-    key = _key(device)
+def _decode_counter_slot(key: tuple[int, int]) -> torch.Tensor | None:
+    """Arrival counters of the one-launch decode for a (device, stream): a slot
+    of the device's pool, which is zeroed and waited for when it is made (every
+    launch leaves its counters zero again), so that a stream that is being
+    captured can take one.  ``None`` -- the decode then takes its two-launch
+    path -- when the pool would have to be made during a capture or has no slot
+    left."""
     slot = _decode_counters.get(key)
     if slot is None:
-        pool = _counter_pools.get(key[0])
-        if pool is None:
-            if torch.cuda.is_current_stream_capturing():
-                return None
-            pool = torch.zeros(_COUNTER_SLOTS, _COUNTER_SLOT_BYTES // 4, dtype=torch.int32, device=device)
-            torch.cuda.current_stream(key[0]).synchronize()
-            _counter_pools[key[0]] = pool
         with _counter_lock:
+            pool = _counter_pools.get(key[0])
+            if pool is None:
+                if torch.cuda.is_current_stream_capturing():
+                    return None
+                pool = torch.zeros(_COUNTER_SLOTS, _COUNTER_SLOT_BYTES // 4, dtype=torch.int32,
+                                   device=torch.device("cuda", key[0]))
+                torch.cuda.current_stream(key[0]).synchronize()
+                _counter_pools[key[0]] = pool
             used = sum(k[0] == key[0] for k in _decode_counters)
             if used >= _COUNTER_SLOTS:
                 return None
             slot = _decode_counters.setdefault(key, pool[used])
-    return slot if nbytes <= _COUNTER_SLOT_BYTES else None
+    return slot
 
 
 def prefill_workspace(device) -> torch.Tensor:
@@ -249,32 +249,22 @@ def paged_decode(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale,
         raise RuntimeError("paged_decode: cache_seqlens and block_table must be int32")
     if block_table.stride(-1) != 1:
         raise RuntimeError("paged_decode: block_table rows must be contiguous")
-    fp8 = k_cache.dtype == torch.float8_e4m3fn
+    kv_dtype = k_cache.dtype
+    fp8 = kv_dtype == torch.float8_e4m3fn
     if out is None:
         out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    o3 = out.squeeze(1) if out.dim() == 4 else out
-    W = block_table.shape[1]
-    config = (ctypes.c_int64 * 4)()
-    check(lib().nq_decode_config(B, hq, hkv, d, W, bs, dtype_code(k_cache.dtype), config), "decode_config")
-    counter_bytes, ns, st, wsb = config
-    counters = None
-    if counter_bytes > 0:    # a small batch: one launch
-        counters = _decode_counter_slot(q.device, counter_bytes)
-        if counters is None:
-            ns, st = decode_plan(B, hq, hkv, W, bs, k_cache.dtype)
-            wsb = lib().nq_decode_workspace_bytes(B, hq, d, ns)
-    ws = decode_workspace(q.device, wsb)
-    args = (ptr(q3), q3.stride(0), q3.stride(1), ptr(k_cache), ptr(v_cache), ptr(block_table),
-            block_table.stride(0), W, ptr(cache_seqlens), ptr(o3), o3.stride(0), o3.stride(1),
-            B, hq, hkv, d, bs, nb, float(softmax_scale), ns, st, ptr(ws), 0 if ws is None else ws.numel(),
-            dtype_code(q.dtype), dtype_code(k_cache.dtype), ptr(k_scale) if fp8 else None,
-            ptr(v_scale) if fp8 else None)
-    g3 = None
+        o_bs, o_hs = hq * d, d
+    else:
+        o3 = out.squeeze(1) if out.dim() == 4 else out
+        o_bs, o_hs = o3.stride(0), o3.stride(1)
+    g_ptr, g_bs, g_hs = None, 0, 0
     if gate is not None:
         require_cuda(gate, what="paged_decode")
         if gate.dtype != q.dtype:
             raise RuntimeError("paged_decode: gate dtype must match q")
         g3 = _gate3(gate, B, hq, d, "paged_decode")
+        g_ptr, g_bs, g_hs = ptr(g3), g3.stride(0), g3.stride(1)
+    new = (None, 0, None, 0, None, -1)
     if k is not None:
         require_cuda(k, v, slot_mapping, what="paged_decode")
         k3 = k.reshape(B, hkv, d) if k.dim() == 4 else k
@@ -282,35 +272,26 @@ def paged_decode(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale,
         for t, what in ((k3, "k"), (v3, "v")):
             if t.shape != (B, hkv, d) or t.stride(-1) != 1 or t.stride(1) != d:
                 raise RuntimeError(f"paged_decode: {what} must be [B, Hkv, D] with contiguous heads")
-        if k3.dtype != v3.dtype or (not fp8 and k3.dtype != k_cache.dtype):
+        if k3.dtype != v3.dtype or (not fp8 and k3.dtype != kv_dtype):
             raise RuntimeError("paged_decode: k/v dtype must match the cache (or be stored into an fp8 cache)")
         if slot_mapping.dtype != torch.int32 or slot_mapping.numel() != B:
             raise RuntimeError("paged_decode: slot_mapping must be int32 [B]")
-    if counters is not None:
-        new = k is not None
-        rc = lib().nq_paged_decode_fused(
+        new = (ptr(k3), k3.stride(0), ptr(v3), v3.stride(0), ptr(slot_mapping), dtype_code(k3.dtype))
+    # The library picks the plan; it asks for a larger workspace once.
+    key = _key(q.device)
+    counters = _decode_counter_slot(key)
+    ws = _workspaces.get(key)
+    need = ctypes.c_int64()
+    while True:
+        rc = lib().nq_paged_decode_auto(
             ptr(q3), q3.stride(0), q3.stride(1), ptr(k_cache), ptr(v_cache), ptr(block_table),
-            block_table.stride(0), W, ptr(cache_seqlens), ptr(k3) if new else None, k3.stride(0) if new else 0,
-            ptr(v3) if new else None, v3.stride(0) if new else 0, ptr(slot_mapping) if new else None,
-            dtype_code(k3.dtype) if new else -1, ptr(o3), o3.stride(0), o3.stride(1),
-            B, hq, hkv, d, bs, nb, float(softmax_scale), ns, st, ptr(ws), 0 if ws is None else ws.numel(),
-            dtype_code(q.dtype), dtype_code(k_cache.dtype), ptr(k_scale) if fp8 else None,
-            ptr(v_scale) if fp8 else None, ptr(g3) if g3 is not None else None,
-            0 if g3 is None else g3.stride(0), 0 if g3 is None else g3.stride(1), ptr(counters),
-            counters.numel() * 4, stream_of(q))
-    elif k is not None:
-        rc = lib().nq_paged_decode_store(
-            ptr(q3), q3.stride(0), q3.stride(1), ptr(k_cache), ptr(v_cache), ptr(block_table),
-            block_table.stride(0), W, ptr(cache_seqlens), ptr(k3), k3.stride(0), ptr(v3), v3.stride(0),
-            ptr(slot_mapping), dtype_code(k3.dtype), ptr(o3), o3.stride(0), o3.stride(1),
-            B, hq, hkv, d, bs, nb, float(softmax_scale), ns, st, ptr(ws), 0 if ws is None else ws.numel(),
-            dtype_code(q.dtype), dtype_code(k_cache.dtype), ptr(k_scale) if fp8 else None,
-            ptr(v_scale) if fp8 else None, ptr(g3) if g3 is not None else None,
-            0 if g3 is None else g3.stride(0), 0 if g3 is None else g3.stride(1), stream_of(q))
-    elif g3 is None:
-        rc = lib().nq_paged_decode(*args, stream_of(q))
-    else:
-        rc = lib().nq_paged_decode_gated(*args, ptr(g3), g3.stride(0), g3.stride(1), stream_of(q))
+            block_table.stride(0), block_table.shape[1], ptr(cache_seqlens), *new, ptr(out), o_bs, o_hs,
+            B, hq, hkv, d, bs, nb, float(softmax_scale), ptr(ws), 0 if ws is None else ws.numel(),
+            dtype_code(q.dtype), dtype_code(kv_dtype), ptr(k_scale) if fp8 else None, ptr(v_scale) if fp8 else None,
+            g_ptr, g_bs, g_hs, ptr(counters), 0 if counters is None else _COUNTER_SLOT_BYTES, need, key[1])
+        if rc != 1:
+            break
+        ws = decode_workspace(q.device, need.value)
     check(rc, "paged_decode")
     return out
 
@@ -375,14 +356,17 @@ def varlen_prefill(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen
             raise RuntimeError("varlen_prefill: gate dtype must match q")
         g3 = _gate3(gate, tq, hq, d, "varlen_prefill")
     gargs = (None, 0, 0) if g3 is None else (ptr(g3), g3.stride(0), g3.stride(1))
-    part_bytes = lib().nq_prefill_split_workspace_bytes(n, tq, int(max_seqlen_q), int(max_seqlen_k), hq, hkv, d)
-    if part_bytes > 0:    # too few work items for the chip: equal key ranges, then a merge
-        parts = _grow(_prefill_parts, _key(q.device), part_bytes, torch.uint8, q.device)
-        rc = lib().nq_varlen_prefill_split(*args, *gargs, tq, ptr(parts), parts.numel(), stream_of(q))
-    elif g3 is None:
-        rc = lib().nq_varlen_prefill(*args, stream_of(q))
-    else:
-        rc = lib().nq_varlen_prefill_gated(*args, *gargs, tq, stream_of(q))
+    # A launch with too few work items for the chip is cut into equal key
+    # ranges and merged; the library asks for the partials' buffer once.
+    key = _key(q.device)
+    parts = _prefill_parts.get(key)
+    need = ctypes.c_int64()
+    while True:
+        rc = lib().nq_varlen_prefill_split(*args, *gargs, tq, ptr(parts), 0 if parts is None else parts.numel(), need,
+                                           key[1])
+        if rc != 1:
+            break
+        parts = _grow(_prefill_parts, key, need.value, torch.uint8, q.device)
     check(rc, "varlen_prefill")
     if _DEBUG_QUEUE:
         _check_queue_zero(ws)
@@ -517,7 +501,8 @@ def gdn_decode(query, key, value, a, b, A_log, dt_bias, state, state_indices, ou
     for t, what in ((q3, "query"), (k3, "key"), (v3, "value")):
         if t.stride(-1) != 1 or t.stride(1) != t.shape[-1] or t.dtype != q3.dtype:
             raise RuntimeError(f"gdn_decode: {what} must be [B, heads, dim] contiguous over (head, dim)")
-    a2, b2 = a.reshape(B, HV), b.reshape(B, HV)
+    a2 = a if a.shape == (B, HV) else a.reshape(B, HV)
+    b2 = b if b.shape == (B, HV) else b.reshape(B, HV)
     if a2.stride(-1) != 1 or b2.stride(-1) != 1 or a2.dtype != q3.dtype or b2.dtype != q3.dtype:
         raise RuntimeError("gdn_decode: a and b must be [B, HV] rows of the query's dtype")
     if A_log.dtype != torch.float32 or dt_bias.dtype != torch.float32:
@@ -562,7 +547,8 @@ def gdn_prefill(query, key, value, a, b, A_log, dt_bias, cu_seqlens, state, stat
     for t, what in ((query, "query"), (key, "key"), (value, "value")):
         if t.stride(-1) != 1 or t.stride(1) != t.shape[-1] or t.dtype != query.dtype or t.shape[0] != T_:
             raise RuntimeError(f"gdn_prefill: {what} must be [T, heads, dim] contiguous over (head, dim)")
-    a2, b2 = a.reshape(T_, HV), b.reshape(T_, HV)
+    a2 = a if a.shape == (T_, HV) else a.reshape(T_, HV)
+    b2 = b if b.shape == (T_, HV) else b.reshape(T_, HV)
     if a2.stride(-1) != 1 or b2.stride(-1) != 1 or a2.dtype != query.dtype or b2.dtype != query.dtype:
         raise RuntimeError("gdn_prefill: a and b must be [T, HV] rows of the query's dtype")
     if A_log.dtype != torch.float32 or dt_bias.dtype != torch.float32:
@@ -583,12 +569,16 @@ def gdn_prefill(query, key, value, a, b, A_log, dt_bias, cu_seqlens, state, stat
             ptr(b2), b2.stride(0), ptr(A_log.contiguous()), ptr(dt_bias.contiguous()), ptr(cu_seqlens), n, ptr(state),
             ptr(state_indices), state.shape[0], 1 if initial_state_from_slot else 0, ptr(out), out.stride(0),
             H, HV, K, V, dtype_code(query.dtype))
-    seg_bytes = lib().nq_gdn_prefill_workspace_bytes(n, T_, HV)
-    if seg_bytes > 0:    # few sequences: cut into segments that run side by side
-        ws = _grow(_gdn_segments, _key(query.device), seg_bytes, torch.uint8, query.device)
-        rc = lib().nq_gdn_prefill_split(*args, T_, ptr(ws), ws.numel(), stream_of(query))
-    else:
-        rc = lib().nq_gdn_prefill(*args, stream_of(query))
+    # Few sequences are cut into segments that run side by side; the library
+    # asks for their states' buffer once.
+    key = _key(query.device)
+    ws = _gdn_segments.get(key)
+    need = ctypes.c_int64()
+    while True:
+        rc = lib().nq_gdn_prefill_split(*args, T_, ptr(ws), 0 if ws is None else ws.numel(), need, key[1])
+        if rc != 1:
+            break
+        ws = _grow(_gdn_segments, key, need.value, torch.uint8, query.device)
     check(rc, "gdn_prefill")
     return out
 
@@ -599,14 +589,15 @@ def gated_rmsnorm(x, gate, weight, eps, out=None):
     ``weight [D]`` float32.  ``out=x`` normalizes in place."""
     require_cuda(x, gate, weight, out, what="gated_rmsnorm")
     d = x.shape[-1]
-    x2, g2 = x.reshape(-1, d), gate.reshape(-1, d)
+    x2 = x if x.dim() == 2 else x.reshape(-1, d)
+    g2 = gate if gate.dim() == 2 and gate.shape[1] == d else gate.reshape(-1, d)
     if x2.stride(-1) != 1 or g2.stride(-1) != 1 or gate.dtype != x.dtype or g2.shape[0] != x2.shape[0]:
         raise RuntimeError("gated_rmsnorm: x and gate must be [..., D] rows of one dtype")
     if weight.dtype != torch.float32 or weight.numel() != d or not weight.is_contiguous():
         raise RuntimeError("gated_rmsnorm: weight must be contiguous float32 [D]")
     if out is None:
         out = torch.empty_like(x)
-    o2 = out.reshape(-1, d)
+    o2 = out if out.dim() == 2 and out.shape[1] == d else out.reshape(-1, d)
     check(lib().nq_gated_rmsnorm(ptr(x2), x2.stride(0), ptr(g2), g2.stride(0), ptr(weight), float(eps), ptr(o2),
                                  o2.stride(0), x2.shape[0], d, dtype_code(x.dtype), stream_of(x)), "gated_rmsnorm")
     return out

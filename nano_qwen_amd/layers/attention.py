@@ -64,12 +64,9 @@ class Attention(nn.Module):
             assert k.stride(1) == head_dim and v.stride(1) == head_dim
             assert k_cache.stride(1) == num_heads * head_dim and v_cache.stride(1) == num_heads * head_dim
             assert context.slot_mapping.numel() == N
-            return kernels.paged_decode(q.unsqueeze(1), k_cache, v_cache,
-                                        cache_seqlens=context.context_lens,
-                                        block_table=context.block_tables, softmax_scale=self.scale,
-                                        k_scale=self.k_scale, v_scale=self.v_scale,
-                                        gate=None if gate is None else gate.unsqueeze(1),
-                                        k=k, v=v, slot_mapping=context.slot_mapping)
+            return kernels.paged_decode(q.unsqueeze(1), k_cache, v_cache, context.context_lens,
+                                        context.block_tables, self.scale, self.k_scale, self.v_scale,
+                                        gate=gate, k=k, v=v, slot_mapping=context.slot_mapping)
         if store:
             store_kvcache(k, v, k_cache, v_cache, context.slot_mapping, self.k_scale, self.v_scale)
         if context.is_prefill:
@@ -86,6 +83,5 @@ class Attention(nn.Module):
             o = kernels.paged_decode(q.unsqueeze(1), k_cache, v_cache,
                                      cache_seqlens=context.context_lens,
                                      block_table=context.block_tables, softmax_scale=self.scale,
-                                     k_scale=self.k_scale, v_scale=self.v_scale,
-                                     gate=None if gate is None else gate.unsqueeze(1))
+                                     k_scale=self.k_scale, v_scale=self.v_scale, gate=gate)
         return o

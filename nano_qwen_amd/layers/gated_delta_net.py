@@ -23,6 +23,11 @@ import torch
 from .. import kernels
 
 
+def _float32(p: torch.Tensor) -> torch.Tensor:
+    p = p.detach()
+    return p if p.dtype == torch.float32 else p.float()
+
+
 def gdn_core(layer, qkv_raw: torch.Tensor, z: torch.Tensor, a: torch.Tensor, b: torch.Tensor,
              state_indices: torch.Tensor, cu_seqlens: torch.Tensor | None = None) -> torch.Tensor:
     """``qkv_raw [T, conv_dim]`` (``in_proj_qkv`` output), ``z [T, value_dim]``,
@@ -34,18 +39,20 @@ def gdn_core(layer, qkv_raw: torch.Tensor, z: torch.Tensor, a: torch.Tensor, b: 
     H, HV = layer.num_k_heads, layer.num_v_heads
     Dk, Dv = layer.head_k_dim, layer.head_v_dim
     kd, vd = H * Dk, HV * Dv
-    w = layer.conv1d.weight.detach().reshape(qkv_raw.shape[1], -1).to(qkv_raw.dtype).contiguous()
+    w = layer.conv1d.weight.detach()
+    if w.dtype != qkv_raw.dtype or not w.is_contiguous():
+        w = w.to(qkv_raw.dtype).contiguous()
     mixed = kernels.gdn_conv1d(qkv_raw, w, layer.conv_states, state_indices, cu_seqlens=cu_seqlens)
-    q = mixed[:, :kd].view(T, H, Dk)
-    k = mixed[:, kd:2 * kd].view(T, H, Dk)
-    v = mixed[:, 2 * kd:].view(T, HV, Dv)
-    A_log = layer.A_log.detach().float()
-    dt_bias = layer.dt_bias.detach().float()
+    q, k, v = mixed.split((kd, kd, vd), dim=1)
+    q, k, v = q.view(T, H, Dk), k.view(T, H, Dk), v.view(T, HV, Dv)
+    A_log = _float32(layer.A_log)
+    dt_bias = _float32(layer.dt_bias)
     if cu_seqlens is None:
         y = kernels.gdn_decode(q, k, v, a, b, A_log, dt_bias, layer.recurrent_states, state_indices)
     else:
         y = kernels.gdn_prefill(q, k, v, a, b, A_log, dt_bias, cu_seqlens, layer.recurrent_states, state_indices)
-    out = y.view(T, vd)
-    kernels.gated_rmsnorm(out.view(-1, Dv), z.reshape(-1, Dv), layer.norm.weight.detach().float().contiguous(),
-                          layer.norm.eps, out=out.view(-1, Dv))
-    return out
+    rows = y.view(-1, Dv)
+    weight = _float32(layer.norm.weight)
+    kernels.gated_rmsnorm(rows, z.reshape(-1, Dv), weight if weight.is_contiguous() else weight.contiguous(),
+                          layer.norm.eps, out=rows)
+    return y.view(T, vd)
