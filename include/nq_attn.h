@@ -12,7 +12,12 @@
  *   - enqueue work asynchronously on that stream: they never allocate, free
  *     or synchronise, so they may be captured into a HIP graph;
  *   - return NQ_OK (0) or a negative status; nq_last_error() then returns a
- *     message for the calling thread.
+ *     message for the calling thread.  (An entry point with a `need` argument
+ *     returns 1, with nothing launched, to ask for a larger workspace.)
+ *
+ * A call may be several launches over its workspace (a main kernel and a
+ * merge).  Host threads that enqueue on one stream with one workspace must
+ * therefore take turns, call by call: the stream orders launches, not calls.
  *
  * Element types are NQ_F32 / NQ_F16 / NQ_BF16 / NQ_FP8_E4M3 (OCP e4m3fn).
  * Strides are in elements of the tensor's own type.

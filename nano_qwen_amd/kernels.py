@@ -22,9 +22,12 @@ import torch
 from . import _lib
 from ._lib import check, dtype_code, lib, ptr, raw_stream, require_cuda, stream_of
 
-# Persistent device buffers of the kernels, one per (device, stream): calls
+# Persistent device buffers of the kernels, one per (device, stream): launches
 # on one stream are ordered, so they may share a buffer; calls on different
-# streams get their own.  A buffer that has to grow is replaced, but the old
+# streams get their own.  A call may be several launches over its buffer (a
+# main kernel and its merge) and ctypes releases the GIL, so a call holds its
+# stream's lock from the buffer's lookup to its last launch: host threads that
+# share a stream take turns.  A buffer that has to grow is replaced, but the old
 # one is kept alive (``_retired``): a HIP graph captured earlier may still
 # hold its address, and replays must keep writing into valid memory.  The
 # tables therefore grow with the number of streams ever used: callers should
@@ -41,7 +44,14 @@ _COUNTER_SLOTS, _COUNTER_SLOT_BYTES = 32, 128 << 10
 _counter_pools: dict[int, torch.Tensor] = {}
 _decode_counters: dict[tuple[int, int], torch.Tensor] = {}
 _counter_lock = threading.Lock()
+# A fixed set of locks, so that streams come and go without leaving any (two
+# streams that share one only wait for each other's host calls).
+_launch_locks = tuple(threading.RLock() for _ in range(64))
 _DEBUG_QUEUE = os.environ.get("NQ_DEBUG_PREFILL_QUEUE", "0") not in ("", "0")
+
+
+def _launch_lock(key: tuple[int, int]):
+    return _launch_locks[hash(key) % len(_launch_locks)]
 
 
 def _key(device) -> tuple[int, int]:
@@ -144,7 +154,9 @@ def decode_workspace(device, nbytes: int) -> torch.Tensor | None:
     """
     if nbytes <= 0:
         return None
-    return _grow(_workspaces, _key(device), nbytes, torch.uint8, device)
+    key = _key(device)
+    with _launch_lock(key):
+        return _grow(_workspaces, key, nbytes, torch.uint8, device)
 
 
 def reserve_decode_workspace(device, max_batch, num_q_heads, num_kv_heads, max_blocks_per_seq, block_size,
@@ -202,8 +214,9 @@ def prefill_workspace(device) -> torch.Tensor:
     never share counters.  With ``NQ_DEBUG_PREFILL_QUEUE=1`` every prefill
     synchronizes and checks that it left them zero.
     """
-    return _grow(_prefill_queues, _key(device), lib().nq_prefill_workspace_bytes(), torch.int32, device,
-                 zero=True)
+    key = _key(device)
+    with _launch_lock(key):
+        return _grow(_prefill_queues, key, lib().nq_prefill_workspace_bytes(), torch.int32, device, zero=True)
 
 
 def _check_queue_zero(ws):
@@ -279,19 +292,21 @@ def paged_decode(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale,
         new = (ptr(k3), k3.stride(0), ptr(v3), v3.stride(0), ptr(slot_mapping), dtype_code(k3.dtype))
     # The library picks the plan; it asks for a larger workspace once.
     key = _key(q.device)
-    counters = _decode_counter_slot(key)
-    ws = _workspaces.get(key)
     need = ctypes.c_int64()
-    while True:
-        rc = lib().nq_paged_decode_auto(
-            ptr(q3), q3.stride(0), q3.stride(1), ptr(k_cache), ptr(v_cache), ptr(block_table),
-            block_table.stride(0), block_table.shape[1], ptr(cache_seqlens), *new, ptr(out), o_bs, o_hs,
-            B, hq, hkv, d, bs, nb, float(softmax_scale), ptr(ws), 0 if ws is None else ws.numel(),
-            dtype_code(q.dtype), dtype_code(kv_dtype), ptr(k_scale) if fp8 else None, ptr(v_scale) if fp8 else None,
-            g_ptr, g_bs, g_hs, ptr(counters), 0 if counters is None else _COUNTER_SLOT_BYTES, need, key[1])
-        if rc != 1:
-            break
-        ws = decode_workspace(q.device, need.value)
+    with _launch_lock(key):
+        counters = _decode_counter_slot(key)
+        ws = _workspaces.get(key)
+        while True:
+            rc = lib().nq_paged_decode_auto(
+                ptr(q3), q3.stride(0), q3.stride(1), ptr(k_cache), ptr(v_cache), ptr(block_table),
+                block_table.stride(0), block_table.shape[1], ptr(cache_seqlens), *new, ptr(out), o_bs, o_hs,
+                B, hq, hkv, d, bs, nb, float(softmax_scale), ptr(ws), 0 if ws is None else ws.numel(),
+                dtype_code(q.dtype), dtype_code(kv_dtype), ptr(k_scale) if fp8 else None,
+                ptr(v_scale) if fp8 else None, g_ptr, g_bs, g_hs, ptr(counters),
+                0 if counters is None else _COUNTER_SLOT_BYTES, need, key[1])
+            if rc != 1:
+                break
+            ws = decode_workspace(q.device, need.value)
     check(rc, "paged_decode")
     return out
 
@@ -359,14 +374,15 @@ def varlen_prefill(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen
     # A launch with too few work items for the chip is cut into equal key
     # ranges and merged; the library asks for the partials' buffer once.
     key = _key(q.device)
-    parts = _prefill_parts.get(key)
     need = ctypes.c_int64()
-    while True:
-        rc = lib().nq_varlen_prefill_split(*args, *gargs, tq, ptr(parts), 0 if parts is None else parts.numel(), need,
-                                           key[1])
-        if rc != 1:
-            break
-        parts = _grow(_prefill_parts, key, need.value, torch.uint8, q.device)
+    with _launch_lock(key):
+        parts = _prefill_parts.get(key)
+        while True:
+            rc = lib().nq_varlen_prefill_split(*args, *gargs, tq, ptr(parts), 0 if parts is None else parts.numel(),
+                                               need, key[1])
+            if rc != 1:
+                break
+            parts = _grow(_prefill_parts, key, need.value, torch.uint8, q.device)
     check(rc, "varlen_prefill")
     if _DEBUG_QUEUE:
         _check_queue_zero(ws)
@@ -572,13 +588,14 @@ def gdn_prefill(query, key, value, a, b, A_log, dt_bias, cu_seqlens, state, stat
     # Few sequences are cut into segments that run side by side; the library
     # asks for their states' buffer once.
     key = _key(query.device)
-    ws = _gdn_segments.get(key)
     need = ctypes.c_int64()
-    while True:
-        rc = lib().nq_gdn_prefill_split(*args, T_, ptr(ws), 0 if ws is None else ws.numel(), need, key[1])
-        if rc != 1:
-            break
-        ws = _grow(_gdn_segments, key, need.value, torch.uint8, query.device)
+    with _launch_lock(key):
+        ws = _gdn_segments.get(key)
+        while True:
+            rc = lib().nq_gdn_prefill_split(*args, T_, ptr(ws), 0 if ws is None else ws.numel(), need, key[1])
+            if rc != 1:
+                break
+            ws = _grow(_gdn_segments, key, need.value, torch.uint8, query.device)
     check(rc, "gdn_prefill")
     return out
 
