@@ -529,10 +529,11 @@ def gdn_decode(query, key, value, a, b, A_log, dt_bias, state, state_indices, ou
         raise RuntimeError("gdn_decode: state_indices must be int32 [B]")
     if out is None:
         out = torch.empty(B, HV, V, dtype=q3.dtype, device=q3.device)
+    A_log, dt_bias = A_log.contiguous(), dt_bias.contiguous()    # held until the launch
     rc = lib().nq_gdn_decode(ptr(q3), q3.stride(0), ptr(k3), k3.stride(0), ptr(v3), v3.stride(0), ptr(a2),
-                             a2.stride(0), ptr(b2), b2.stride(0), ptr(A_log.contiguous()),
-                             ptr(dt_bias.contiguous()), ptr(state), ptr(state_indices), state.shape[0],
-                             ptr(out), out.stride(0), B, H, HV, K, V, dtype_code(q3.dtype), stream_of(q3))
+                             a2.stride(0), ptr(b2), b2.stride(0), ptr(A_log), ptr(dt_bias), ptr(state),
+                             ptr(state_indices), state.shape[0], ptr(out), out.stride(0), B, H, HV, K, V,
+                             dtype_code(q3.dtype), stream_of(q3))
     check(rc, "gdn_decode")
     return out
 
@@ -581,8 +582,9 @@ def gdn_prefill(query, key, value, a, b, A_log, dt_bias, cu_seqlens, state, stat
     for t, what in ((query, "query"), (key, "key"), (value, "value"), (a2, "a"), (b2, "b")):
         if _overlaps(out, t):
             raise RuntimeError(f"gdn_prefill: out must not overlap {what}")
+    A_log, dt_bias = A_log.contiguous(), dt_bias.contiguous()    # held until the launch
     args = (ptr(query), query.stride(0), ptr(key), key.stride(0), ptr(value), value.stride(0), ptr(a2), a2.stride(0),
-            ptr(b2), b2.stride(0), ptr(A_log.contiguous()), ptr(dt_bias.contiguous()), ptr(cu_seqlens), n, ptr(state),
+            ptr(b2), b2.stride(0), ptr(A_log), ptr(dt_bias), ptr(cu_seqlens), n, ptr(state),
             ptr(state_indices), state.shape[0], 1 if initial_state_from_slot else 0, ptr(out), out.stride(0),
             H, HV, K, V, dtype_code(query.dtype))
     # Few sequences are cut into segments that run side by side; the library

@@ -515,3 +515,28 @@ def test_gdn_prefill_segments(cuda, lens, H, HV, kind, from_slot, monkeypatch):
         off[how] = [float((x.double() - y).norm() / y.norm()) for x, y in ((out, ref), (state[live], ref_state[live]))]
     print(f"[gdn] {lens} {kind}: error of outputs and states {off}", flush=True)
     assert all(s <= 1.1 * w for s, w in zip(off["segments"], off["whole"]))
+    if "slow" in kind:
+        assert not torch.equal(outs["segments"], outs["whole"])
+
+
+@pytest.mark.parametrize("prefill", [False, True])
+def test_gdn_strided_parameters(cuda, prefill):
+    """A_log and dt_bias as columns of one tensor: their contiguous copies live
+    until the launch (a copy freed before it is the next copy's memory)."""
+    n = 70 if prefill else 3
+    c = _prefill_inputs([n] if prefill else [1] * n, 4, 8, seed=5, slots=4)
+    d = {k: v.to(cuda) for k, v in c.items()}
+    both = torch.stack([d["A_log"], d["dt"]], 1)
+    outs = []
+    for A_log, dt in ((d["A_log"], d["dt"]), (both[:, 0], both[:, 1])):
+        assert A_log.is_contiguous() == (not outs)
+        state = d["state"].clone()
+        if prefill:
+            out = kernels.gdn_prefill(d["q"], d["k"], d["v"], d["a"], d["b"], A_log, dt, d["cu"], state,
+                                      torch.zeros(1, dtype=torch.int32, device=cuda))
+        else:
+            out = kernels.gdn_decode(d["q"], d["k"], d["v"], d["a"], d["b"], A_log, dt, state,
+                                     torch.arange(n, dtype=torch.int32, device=cuda))
+        torch.cuda.synchronize()
+        outs.append((out, state))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
