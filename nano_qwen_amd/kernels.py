@@ -200,6 +200,9 @@ def _decode_counter_slot(key: tuple[int, int]) -> torch.Tensor | None:
             used = sum(k[0] == key[0] for k in _decode_counters)
             if used >= _COUNTER_SLOTS:
                 return None
+            # the pool was made on another stream: released, it is not handed
+            # out again before this stream's launches have ended
+            pool.record_stream(torch.cuda.current_stream(key[0]))
             slot = _decode_counters.setdefault(key, pool[used])
     return slot
 

@@ -113,3 +113,27 @@ def test_fused_decode_streams_have_their_own_counters(cuda):
     assert all(torch.equal(o, want) for o in outs)
     slots = [kernels._decode_counters[(0, s.cuda_stream)].data_ptr() for s in streams]
     assert slots[0] != slots[1]
+
+
+def test_released_counters_outlive_their_streams_work(cuda):
+    """The pool is made on one stream and used on others: released while another
+    stream's decode is still to run, its memory is not handed out before that."""
+    case = make_decode_case("cfg2", seed=9, device=cuda, batch=2, ctx=(700, 700), hq=8, hkv=2)
+    args = (case["q"].unsqueeze(1), case["k_cache"], case["v_cache"], case["context_lens"], case["block_tables"],
+            case["scale"])
+    want = kernels.paged_decode(*args)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        kernels.paged_decode(*args)
+        torch.cuda.synchronize()
+        pool = kernels._counter_pools[0]
+        where, shape = pool.data_ptr(), pool.shape
+        torch.cuda._sleep(1_000_000_000)
+        out = kernels.paged_decode(*args)
+    del pool
+    kernels.release_workspaces()
+    taken = [torch.full(shape, 3, dtype=torch.int32, device=cuda) for _ in range(100)]
+    assert not side.query()    # still to run
+    assert all(t.data_ptr() != where for t in taken)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
