@@ -47,6 +47,9 @@ enum nq_dtype { NQ_F32 = 0, NQ_F16 = 1, NQ_BF16 = 2, NQ_FP8_E4M3 = 3 };
 /* Version of this ABI (NQ_ABI_VERSION). */
 int nq_abi_version(void);
 
+/* The id of the capture that `stream` is in (0: none, or not known). */
+int64_t nq_capture_id(void *stream);
+
 /* Message for the last non-zero status returned on this thread. */
 const char *nq_last_error(void);
 
@@ -213,8 +216,11 @@ int nq_paged_decode_store(const void *q, int64_t q_batch_stride, int64_t q_head_
  * k_new (no store when null) and gate optional, whose splits are merged by the
  * workgroup of each (sequence, kv head) that finishes last.  counters: 64
  * bytes of device memory per (sequence, kv head), 64-byte aligned, zero before
- * the first call that uses them; every completed call leaves them zero.  Calls that overlap may
- * share neither them nor the workspace.  num_splits and split_tokens as
+ * the first call that uses them; every completed call leaves them zero.  Calls
+ * that overlap may share neither them nor the workspace: counters that an overlap
+ * left nonzero spoil the calls after it too.  A capture had better zero its
+ * counters ahead of its first call (nq_capture_id tells a new capture), so that
+ * replays that overlapped spoil no later one.  num_splits and split_tokens as
  * nq_decode_config gives them (any plan that nq_paged_decode accepts is).
  */
 int nq_paged_decode_fused(const void *q, int64_t q_batch_stride, int64_t q_head_stride,

@@ -56,6 +56,7 @@ _SIGS = {
                                   c_void_p, c_int, c_int, c_void_p, c_int64, c_int, c_int64, c_void_p,
                                   c_int64, c_int64, c_int, c_int, c_int, c_int, c_int, c_float, c_int,
                                   c_int, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
+    "nq_capture_id": (c_int64, [c_void_p]),
     "nq_decode_config": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int, POINTER(c_int64)]),
     "nq_paged_decode_auto": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_int,
                                      c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int, c_void_p,

@@ -39,3 +39,13 @@ int device_cus() {
 extern "C" int nq_abi_version(void) { return NQ_ABI_VERSION; }
 
 extern "C" const char *nq_last_error(void) { return nq::g_last_error; }
+
+extern "C" int64_t nq_capture_id(void *stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(static_cast<hipStream_t>(stream), &status, &id) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  return status == hipStreamCaptureStatusActive ? static_cast<int64_t>(id) : 0;
+}

@@ -39,10 +39,12 @@ _prefill_parts: dict[tuple[int, int], torch.Tensor] = {}
 _gdn_segments: dict[tuple[int, int], torch.Tensor] = {}
 _retired: list[torch.Tensor] = []
 # Zeroed arrival counters of the one-launch decode: a pool per device, a slot
-# per (device, stream).
-_COUNTER_SLOTS, _COUNTER_SLOT_BYTES = 32, 128 << 10
+# per (device, stream) and a second one for what is captured on that stream,
+# with the id of the last capture that zeroed it.
+_COUNTER_SLOTS, _COUNTER_SLOT_BYTES = 64, 128 << 10
 _counter_pools: dict[int, torch.Tensor] = {}
 _decode_counters: dict[tuple[int, int], torch.Tensor] = {}
+_capture_counters: dict[tuple[int, int], tuple[int, torch.Tensor]] = {}
 _counter_lock = threading.Lock()
 # A fixed set of locks, so that streams come and go without leaving any (two
 # streams that share one only wait for each other's host calls).
@@ -86,7 +88,8 @@ def release_workspaces(device=None) -> int:
     at zero again)."""
     idx = None if device is None else _key(device)[0]
     n = 0
-    for table in (_workspaces, _prefill_queues, _prefill_parts, _gdn_segments, _decode_counters):
+    for table in (_workspaces, _prefill_queues, _prefill_parts, _gdn_segments, _decode_counters,
+                  _capture_counters):
         for key in [k for k in table if idx is None or k[0] == idx]:
             del table[key]
             n += 1
@@ -179,31 +182,52 @@ def reserve_decode_workspace(device, max_batch, num_q_heads, num_kv_heads, max_b
     return need
 
 
-def _decode_counter_slot(key: tuple[int, int]) -> torch.Tensor | None:
-    """Arrival counters of the one-launch decode for a (device, stream): a slot
-    of the device's pool, which is zeroed and waited for when it is made (every
-    launch leaves its counters zero again), so that a stream that is being
-    captured can take one.  ``None`` -- the decode then takes its two-launch
-    path -- when the pool would have to be made during a capture or has no slot
-    left."""
-    slot = _decode_counters.get(key)
-    if slot is None:
-        with _counter_lock:
-            pool = _counter_pools.get(key[0])
-            if pool is None:
-                if torch.cuda.is_current_stream_capturing():
-                    return None
-                pool = torch.zeros(_COUNTER_SLOTS, _COUNTER_SLOT_BYTES // 4, dtype=torch.int32,
-                                   device=torch.device("cuda", key[0]))
-                torch.cuda.current_stream(key[0]).synchronize()
-                _counter_pools[key[0]] = pool
-            used = sum(k[0] == key[0] for k in _decode_counters)
-            if used >= _COUNTER_SLOTS:
+def _take_counter_slot(key: tuple[int, int], capturing: bool) -> torch.Tensor | None:
+    """A slot of the device's pool, which is zeroed and waited for when it is
+    made.  ``None`` -- the decode then takes its two-launch path -- when the pool
+    would have to be made during a capture or has no slot left."""
+    with _counter_lock:
+        pool = _counter_pools.get(key[0])
+        if pool is None:
+            if capturing:
                 return None
-            # the pool was made on another stream: released, it is not handed
-            # out again before this stream's launches have ended
-            pool.record_stream(torch.cuda.current_stream(key[0]))
-            slot = _decode_counters.setdefault(key, pool[used])
+            pool = torch.zeros(_COUNTER_SLOTS, _COUNTER_SLOT_BYTES // 4, dtype=torch.int32,
+                               device=torch.device("cuda", key[0]))
+            torch.cuda.current_stream(key[0]).synchronize()
+            _counter_pools[key[0]] = pool
+        used = sum(k[0] == key[0] for table in (_decode_counters, _capture_counters) for k in table)
+        if used >= _COUNTER_SLOTS:
+            return None
+        # the pool was made on another stream: released, it is not handed
+        # out again before this stream's launches have ended
+        pool.record_stream(torch.cuda.current_stream(key[0]))
+        if capturing:
+            _capture_counters[key] = 0, pool[used]
+        else:
+            _decode_counters[key] = pool[used]
+        return pool[used]
+
+
+def _decode_counter_slot(key: tuple[int, int]) -> torch.Tensor | None:
+    """Arrival counters of the one-launch decode for a (device, stream).  Every
+    launch leaves its counters zero again, so those of a stream's own launches
+    stay in order.  Graphs captured on one stream may be replayed on several,
+    and replays that overlap spoil their common counters: captured launches
+    have a slot of their own, and a capture's first decode records its zeroing,
+    so that the damage ends with those replays.  Called with the stream's
+    launch lock held."""
+    if not torch.cuda.is_current_stream_capturing():
+        slot = _decode_counters.get(key)
+        return slot if slot is not None else _take_counter_slot(key, False)
+    last, slot = _capture_counters.get(key, (0, None))
+    if slot is None:
+        slot = _take_counter_slot(key, True)
+        if slot is None:
+            return None
+    now = lib().nq_capture_id(key[1])
+    if now != last or now == 0:
+        slot.zero_()    # a fill kernel
+        _capture_counters[key] = now, slot
     return slot
 
 

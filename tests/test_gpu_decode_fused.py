@@ -115,6 +115,38 @@ def test_fused_decode_streams_have_their_own_counters(cuda):
     assert slots[0] != slots[1]
 
 
+def test_fused_decode_spoiled_counters_do_not_last(cuda):
+    """Counters that an overlap of two replays left nonzero (every slot of the
+    pool but the eager stream's): the graphs' next replays are right, and leave
+    theirs zero."""
+    cases = [make_decode_case("cfg2", seed=s, device=cuda, batch=2, ctx=(700, 700), hq=8, hkv=2) for s in (5, 6)]
+    args = [(c["q"].unsqueeze(1), c["k_cache"], c["v_cache"], c["context_lens"], c["block_tables"], c["scale"])
+            for c in cases]
+    assert all(map(_fused, cases))
+    want = [kernels.paged_decode(*a) for a in args]
+    torch.cuda.synchronize()
+    graphs, outs = [], []
+    for a in args:    # as a runner captures: torch's own capture stream, several decodes each
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            outs.append([kernels.paged_decode(*a) for _ in range(3)])
+        graphs.append(graph)
+    pool = kernels._counter_pools[0]
+    eager = kernels._decode_counters[(0, torch.cuda.current_stream().cuda_stream)]
+    for _ in range(3):
+        for graph, got, w in zip(graphs, outs, want):
+            pool.fill_(7)
+            eager.zero_()
+            for o in got:
+                o.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(o, w) for o in got)
+            assert torch.equal(kernels.paged_decode(*args[0]), want[0])
+    pool.zero_()
+    torch.cuda.synchronize()
+
+
 def test_released_counters_outlive_their_streams_work(cuda):
     """The pool is made on one stream and used on others: released while another
     stream's decode is still to run, its memory is not handed out before that."""
