@@ -284,6 +284,14 @@ struct DecodeWave {
   }
 };
 
+// log2-sum-exp of a piece with row maximum m and row sum L, in its workspace
+// slot.  -inf marks a piece without tokens, whose slot may be stale; a piece
+// with tokens never has it: one whose keys all have no weight (missing blocks,
+// scores of -inf) gets the lowest finite value, below any score, and the NaN of
+// a NaN sum stays, so that the merge passes it on.
+constexpr float kNoWeight = -__FLT_MAX__;
+__device__ __forceinline__ float piece_lse(float m, float L) { return L == 0.f ? kNoWeight : m + __log2f(L); }
+
 // The work of one wave on one piece of a sequence: kv head kvh of sequence
 // b over tokens [t_begin, t_end) (t_begin % 32 == 0, at most 63 blocks).
 // STRIDE 1: the wave takes all 32-token steps; a piece that is the whole
@@ -463,7 +471,7 @@ __device__ __forceinline__ void decode_piece(const DecodeArgs &a, uint8_t *tile,
     float *wp = a.ws_o + idx * D;
 #pragma unroll
     for (int j = 0; j < Gm::NJ; ++j) *reinterpret_cast<f32x4 *>(wp + 16 * j + 4 * g) = o[j] * inv;
-    if (g == 0) a.ws_lse[idx] = (L > 0.f) ? m_run + __log2f(L) : kNegInf;
+    if (g == 0) a.ws_lse[idx] = piece_lse(m_run, L);
   }
 }
 
@@ -578,13 +586,15 @@ __device__ __forceinline__ void merge_loop(const DecodeArgs &a, int first, int s
         }
       }
     }
-    float mc = kNegInf;
+    float mc = kNegInf;  // of a NaN and others: the others'
+    bool some = false;
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
+      some |= l[u] != kNegInf;
       if (c0 + u * step >= 1) any |= l[u] != kNegInf;
       mc = fmaxf(mc, l[u]);
     }
-    if (mc == kNegInf) continue;  // every piece of the chunk is empty
+    if (!some) continue;  // every piece of the chunk is empty
     const float mn = fmaxf(M, mc);
     if (M != kNegInf) {
       const float f = __builtin_amdgcn_exp2f(M - mn);
@@ -621,15 +631,15 @@ __device__ __forceinline__ bool merge_pieces(const DecodeArgs &a, int n, Row row
       float mx = part_m[0];
 #pragma unroll
       for (int u = 1; u < GR; ++u) mx = fmaxf(mx, part_m[u]);
+      if (mx == kNegInf) mx = 0.f;  // no piece, or only NaN
       W = 0.f;
       acc = f32x4{0, 0, 0, 0};
-      if (mx != kNegInf)
 #pragma unroll
-        for (int u = 0; u < GR; ++u) {
-          const float f = __builtin_amdgcn_exp2f(part_m[u] - mx);  // 0 for a group without pieces
-          W += part_w[u] * f;
-          acc += *reinterpret_cast<const f32x4 *>(&part[u][4 * d4]) * f;
-        }
+      for (int u = 0; u < GR; ++u) {
+        const float f = __builtin_amdgcn_exp2f(part_m[u] - mx);  // 0 for a group without pieces
+        W += part_w[u] * f;
+        acc += *reinterpret_cast<const f32x4 *>(&part[u][4 * d4]) * f;
+      }
     }
   }
   later = any;
@@ -711,8 +721,7 @@ void paged_decode_fused_kernel(const DecodeArgs a) {
       const int64_t idx = (static_cast<int64_t>(b) * a.Hq + head) * a.num_splits + split;
       store_shared4(a.ws_o + idx * D + 4 * d4, acc);
       if (d4 == 0)
-        __hip_atomic_store(a.ws_lse + idx, L > 0.f ? M + __log2f(L) : kNegInf, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(a.ws_lse + idx, piece_lse(M, L), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
   if (n_split == 1) return;
