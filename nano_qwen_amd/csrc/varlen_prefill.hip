@@ -1575,15 +1575,17 @@ __global__ __launch_bounds__(64 * S::NW * S::QS) void prefill_merge_kernel(const
     float mc = M;
 #pragma unroll
     for (int i = 0; i < kChunk; ++i) mc = fmaxf(mc, l[i]);
-    if (mc == kNegInf) mc = 0.f;  // no piece has a visible key yet: weights 0
-    const float f = __builtin_amdgcn_exp2f(M - mc);
+    // No piece has a visible key yet: weights 0, and a maximum that stays -inf,
+    // so that later pieces are weighed against their own.
+    const float mu = mc == kNegInf ? 0.f : mc;
+    const float f = __builtin_amdgcn_exp2f(M - mu);
     W *= f;
 #pragma unroll
     for (int j = 0; j < kMergeJ; ++j) acc[j] *= f;
 #pragma unroll
     for (int i = 0; i < kChunk; ++i)
       if (sl[i] >= 0) {
-        const float wt = __builtin_amdgcn_exp2f(l[i] - mc);
+        const float wt = __builtin_amdgcn_exp2f(l[i] - mu);
         W += wt;
 #pragma unroll
         for (int j = 0; j < kMergeJ; ++j) acc[j] += p[i][j] * wt;

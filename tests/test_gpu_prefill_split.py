@@ -10,7 +10,7 @@ import torch
 from nano_qwen_amd import kernels
 from nano_qwen_amd._lib import lib
 from oracle.inputs import make_prefill_case
-from tests.parity import TOL_BF16, TOL_FP8
+from tests.parity import TOL_BF16, TOL_FP8, assert_close, f64
 from tests.test_gpu_prefill import check, run_step
 
 pytestmark = pytest.mark.gpu
@@ -69,3 +69,38 @@ def test_prefill_ranges_gate_and_reuse(cuda):
     want = out * torch.sigmoid(gate)
     off = (got.view(torch.int16).int() - want.view(torch.int16).int()).abs()
     assert int(off.max()) <= 1 and float((off > 0).float().mean()) <= 1e-3
+
+
+@pytest.mark.parametrize("lq,d", [(1, 128), (40, 128), (1, 256), (40, 256)])
+def test_prefill_ranges_invisible_front(cuda, lq, d):
+    """The first half of the table missing: an item's first pieces hold no
+    visible key, more of them than the merge reads at once.  The visible keys
+    all score -196 (log2), so a row is the mean of the values it sees."""
+    case = make_prefill_case("cfg3", seed=7, device=cuda, nseq=1, lq=(lq, lq), prefix_blocks=(31, 31), hq=8, hkv=2, d=d)
+    assert _ranges(case)
+    hidden = 16 * case["block_size"]
+    case["q"].fill_(1.0)
+    case["k_cache"].fill_(-196.0 / (case["scale"] * d * 1.4427))
+    case["block_tables"][0, :16] = -1
+    out = kernels.varlen_prefill(case["q"], case["k_cache"], case["v_cache"], case["cu_seqlens_q"], case["cu_seqlens_k"],
+                                 case["max_seqlen_q"], case["max_seqlen_k"], case["scale"],
+                                 block_table=case["block_tables"])
+    v = case["v_cache"][case["block_tables"][0, 16:].long()].flatten(0, 1)[:case["lk"][0] - hidden].double()
+    upto = torch.arange(v.shape[0] - lq, v.shape[0], device=cuda)
+    want = (v.cumsum(0)[upto] / (upto + 1).view(-1, 1, 1)).repeat_interleave(4, 1)
+    assert_close(f64(out), f64(want), **TOL_BF16, what="visible half")
+
+
+@pytest.mark.parametrize("d", [128, 256])
+def test_prefill_ranges_nan_key(cuda, d):
+    """A NaN key reaches its heads' rows whichever piece holds it, beside pieces without visible keys too."""
+    case = make_prefill_case("cfg3", seed=8, device=cuda, nseq=1, lq=(20, 20), prefix_blocks=(31, 31), hq=8, hkv=2, d=d)
+    assert _ranges(case)
+    case["block_tables"][0, 4:8] = -1
+    for t in (3, 2300, 7700):
+        k = case["k_cache"].clone()
+        k[case["block_tables"][0, t // 256], t % 256, 1, 9] = float("nan")
+        out = kernels.varlen_prefill(case["q"], k, case["v_cache"], case["cu_seqlens_q"], case["cu_seqlens_k"],
+                                     case["max_seqlen_q"], case["max_seqlen_k"], case["scale"],
+                                     block_table=case["block_tables"])
+        assert out[:, 4:].isnan().all() and not out[:, :4].isnan().any()
