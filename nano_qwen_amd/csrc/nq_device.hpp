@@ -261,6 +261,9 @@ __device__ inline void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
   __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
 }
+// Waits until this wave's stores have completed, and keeps the compiler from
+// moving memory accesses across (the builtin above is no barrier to it).
+__device__ inline void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 __device__ inline void wait_lgkmcnt0() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 // Workgroup barrier without the memory-model fence __syncthreads() implies
 // (which would wait for every outstanding load, including in-flight DMA).

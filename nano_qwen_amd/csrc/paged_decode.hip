@@ -725,7 +725,7 @@ void paged_decode_fused_kernel(const DecodeArgs a) {
     }
   }
   if (n_split == 1) return;
-  wait_vmcnt<0>();  // this wave's device-scope stores have completed
+  wait_stores();    // this wave's device-scope stores have completed
   __syncthreads();  // and every other wave's
   if (threadIdx.x == 0) {
     unsigned *c = a.counters + (static_cast<int64_t>(b) * a.Hkv + kvh) * (kCounterBytes / 4);
