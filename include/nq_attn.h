@@ -395,8 +395,9 @@ int nq_varlen_prefill_split(const void *q, int64_t q_row_stride, int64_t q_head_
                             int64_t *need, void *stream);
 
 /* Bytes of split_workspace with which nq_varlen_prefill_split cuts a launch of
- * these sizes into equal ranges; 0: it would not (decided from the sizes and
- * the current device alone). */
+ * these sizes into equal ranges (at head_dim 256 16-bit K/V is cut up to fewer
+ * work items than fp8, for which this answers); 0: it would not (decided from
+ * the sizes and the current device alone). */
 int64_t nq_prefill_split_workspace_bytes(int num_seqs, int64_t total_q, int max_seqlen_q, int max_seqlen_k,
                                          int num_q_heads, int num_kv_heads, int head_dim);
 

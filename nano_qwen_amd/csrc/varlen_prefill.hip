@@ -1615,6 +1615,18 @@ __global__ __launch_bounds__(64 * S::NW * S::QS) void prefill_merge_kernel(const
 // dynamic queue balances by itself: 16 prompts with 7.4 items per workgroup
 // 289 us whole, 323 as ranges; 6 at head_dim 256 with 5.2 items 303 and 391; at
 // 3.9 items (4 kv heads) 178 and 175.
+//
+// Whole items of one sequence that run in step share its K/V tiles in L2; cut
+// ones start at different keys and read them again.  At head_dim 256 over 16-bit
+// K/V that costs more than the even split gains for several sequences with more
+// than 1.5 items per workgroup when cached keys prevail (items of nearly one
+// cost), 1.75 when not.  Whole and ranges at 4 kv heads: 16 of 75-300 tokens
+// behind 8192 (at most 1.80 items) 590 and 854 us, behind 512 80 and 96; 8 of
+// 150-600 behind 8192 (1.64) 548 and 723; 4 of 280-1111 behind 8192 (1.73) 562 and
+// 656, without a prefix 83 and 77; 12 of 639 at 2 kv heads without (1.88) 66 and
+// 80; but 4 of 600 behind 8192 (1.19) 530 and 478.  Over fp8 K/V, half the bytes,
+// the first 710 and 672, the third 733 and 615; at head_dim 128 two of 684 launches
+// were more than 2% slower as ranges (567 and 623, 532 and 544).
 template <int D, class S>
 struct RangePlan {
   static constexpr int64_t kSlotO = static_cast<int64_t>(S::NW) * S::QS * (D / 16) * 1024;
@@ -1628,12 +1640,14 @@ struct RangePlan {
     const int64_t w = rl > 0 ? 1 : (U >= 8 ? (n_y + 7) / 8 : n_y);
     return num_seqs * static_cast<int64_t>((n_qtiles + (1 << rl) - 1) >> rl) * w;
   }
-  static bool use(int num_seqs, int64_t total_q, int max_seqlen_q, int max_seqlen_k, int n_y, int G4) {
+  static bool use(int num_seqs, int64_t total_q, int max_seqlen_q, int max_seqlen_k, int n_y, int G4, bool fp8) {
     const int rows = S::ITEM_ROWS / G4;
     const int n_qtiles = (max_seqlen_q + rows - 1) / rows;
     const int64_t items = std::min<int64_t>((total_q + rows - 1) / rows + num_seqs, static_cast<int64_t>(num_seqs) * n_qtiles) * n_y;
+    int quarters = 4 * kRangeWaves;
+    if (D == 256 && !fp8 && num_seqs > 1) quarters = 2LL * max_seqlen_k >= 3LL * max_seqlen_q ? 6 : 7;
     return num_seqs <= kMaxSeqs && entries(num_seqs, n_qtiles, n_y) < S::MAX_ITEMS &&
-           max_seqlen_k >= kRangeKeys && items < kRangeWaves * grid();
+           max_seqlen_k >= kRangeKeys && 4 * items < quarters * grid();
   }
 };
 
@@ -1648,7 +1662,7 @@ int launch_prefill_dma(PrefillArgs a, int64_t total_q, uint8_t *split_ws, int64_
   a.pin = U >= 8;
   using RP = RangePlan<D, S>;
   if (split_ws && split_bytes >= RP::bytes() &&
-      RP::use(a.num_seqs, total_q, a.max_seqlen_q, a.max_seqlen_k, a.Hkv * a.quads, a.G4)) {
+      RP::use(a.num_seqs, total_q, a.max_seqlen_q, a.max_seqlen_k, a.Hkv * a.quads, a.G4, FP8)) {
     const int grid = RP::grid();
     a.rep_log2 = shared_slots_log2(a.Hkv * a.quads);
     if (a.rep_log2 > 0) a.pin = 1;
@@ -1853,20 +1867,25 @@ extern "C" int nq_varlen_prefill_gated(
                              workspace_bytes, gate, gate_row_stride, gate_head_stride, total_q, nullptr, 0, stream);
 }
 
-extern "C" int64_t nq_prefill_split_workspace_bytes(int num_seqs, int64_t total_q, int max_seqlen_q, int max_seqlen_k,
-                                                    int num_q_heads, int num_kv_heads, int head_dim) {
+static int64_t prefill_split_bytes(int num_seqs, int64_t total_q, int max_seqlen_q, int max_seqlen_k, int num_q_heads,
+                                   int num_kv_heads, int head_dim, bool fp8) {
   if (num_seqs <= 0 || total_q <= 0 || max_seqlen_q <= 0 || max_seqlen_k <= 0 || num_kv_heads <= 0 ||
       num_q_heads < num_kv_heads || num_q_heads % num_kv_heads != 0)
     return 0;
   const int G = num_q_heads / num_kv_heads, G4 = G < 4 ? G : 4, n_y = num_kv_heads * (G < 4 ? 1 : G / 4);
   if ((G > 4 && G % 4 != 0) || G == 3) return 0;
   if (head_dim == 128)
-    return RangePlan<128, ShapeC>::use(num_seqs, total_q, max_seqlen_q, max_seqlen_k, n_y, G4)
+    return RangePlan<128, ShapeC>::use(num_seqs, total_q, max_seqlen_q, max_seqlen_k, n_y, G4, fp8)
                ? RangePlan<128, ShapeC>::bytes() : 0;
   if (head_dim == 256)
-    return RangePlan<256, ShapeD>::use(num_seqs, total_q, max_seqlen_q, max_seqlen_k, n_y, G4)
+    return RangePlan<256, ShapeD>::use(num_seqs, total_q, max_seqlen_q, max_seqlen_k, n_y, G4, fp8)
                ? RangePlan<256, ShapeD>::bytes() : 0;
   return 0;
+}
+
+extern "C" int64_t nq_prefill_split_workspace_bytes(int num_seqs, int64_t total_q, int max_seqlen_q, int max_seqlen_k,
+                                                    int num_q_heads, int num_kv_heads, int head_dim) {
+  return prefill_split_bytes(num_seqs, total_q, max_seqlen_q, max_seqlen_k, num_q_heads, num_kv_heads, head_dim, true);
 }
 
 extern "C" int nq_varlen_prefill_split(
@@ -1879,8 +1898,8 @@ extern "C" int nq_varlen_prefill_split(
     int64_t gate_head_stride, int64_t total_q, void *split_workspace, int64_t split_workspace_bytes, int64_t *need,
     void *stream) {
   if (need) {
-    const int64_t bytes = nq_prefill_split_workspace_bytes(num_seqs, total_q, max_seqlen_q, max_seqlen_k, num_q_heads,
-                                                           num_kv_heads, head_dim);
+    const int64_t bytes = prefill_split_bytes(num_seqs, total_q, max_seqlen_q, max_seqlen_k, num_q_heads, num_kv_heads,
+                                              head_dim, kv_dtype == NQ_FP8_E4M3);
     if (bytes > 0 && (!split_workspace || split_workspace_bytes < bytes)) {
       *need = bytes;
       return 1;

@@ -3,9 +3,13 @@
 exactly once, a cut falls on a cache-block boundary, each range holds at most
 one continued and one continuing item, and the merge's walk from an item's
 first piece meets exactly its other pieces."""
+import ctypes
 import random
 
 import pytest
+import torch
+
+from nano_qwen_amd._lib import dtype_code, lib
 
 KEYS, ITEM, MIN = 32, 8, 2
 
@@ -113,3 +117,35 @@ def test_ranges_cover_and_chain(n_y, rows, n_wg, tpb):
         pin = pin or rep > 1
         for x in range(8) if pin else (0,):
             check_queue(Queue(x, lq, lk, n_y, rows, pin, rep, n_wg if pin else 8 * n_wg, tpb, trial != 4))
+
+
+def _cut(n, total_q, max_q, max_k, hq, hkv, d, kv):
+    """Whether the library would cut such a launch: it asks for the partials' buffer, with nothing launched."""
+    need = ctypes.c_int64()
+    rc = lib().nq_varlen_prefill_split(None, 0, 0, None, None, 0, None, None, max_q, max_k, None, 0, 0, 0, None, 0, 0, n,
+                                       hq, hkv, d, 256, 1.0, 1, dtype_code(torch.bfloat16), dtype_code(kv), None, None,
+                                       None, 0, None, 0, 0, total_q, None, 0, need, None)
+    assert rc == 1 and need.value > 0 or rc < 0 and need.value == 0
+    return rc == 1
+
+
+BF16, FP8 = torch.bfloat16, torch.float8_e4m3fn
+
+
+@pytest.mark.parametrize("n,total_q,max_q,prefix,d,kv,cut", [
+    (16, 3100, 300, 8192, 256, BF16, False),    # 1.7 items per workgroup of nearly one cost: they share K/V in L2
+    (16, 3100, 300, 512, 256, BF16, False),
+    (16, 3100, 300, 8192, 256, FP8, True),
+    (16, 3100, 300, 8192, 128, BF16, True),
+    (8, 3000, 600, 8192, 256, BF16, False),
+    (4, 3300, 1111, 8192, 256, BF16, False),
+    (4, 3300, 1111, 0, 256, BF16, True),        # causal from the first key: costs differ
+    (12, 7668, 639, 0, 256, BF16, False),
+    (4, 2400, 600, 8192, 256, BF16, True),      # 1.2 items
+    (1, 3600, 3600, 8192, 256, BF16, True),     # one sequence
+    (4, 800, 300, 6000, 256, BF16, True),
+])
+def test_which_launches_are_cut(n, total_q, max_q, prefix, d, kv, cut):
+    hq, hkv = (16, 4) if d == 256 else (32, 8)
+    hkv = 2 if n == 12 else hkv
+    assert _cut(n, total_q, max_q, max_q + prefix, 4 * hkv, hkv, d, kv) == cut
