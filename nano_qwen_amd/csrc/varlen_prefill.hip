@@ -121,10 +121,18 @@ __device__ inline int swz8(int row) {
 // tokens, 4 kv heads of 256, 349 -> 255 us; 16 prompts of 256-2048 behind
 // prefixes, 4 kv heads of 128, 215 -> 178 us.  A slot's K/V is then read into
 // 2, 4 or 8 L2s instead of one.
-inline int shared_slots_log2(int n_y) {
+//
+// 8 groups or more stay whole where that gains nothing: with fewer than two
+// query tiles for each XCD of a slot some XCDs would get one or none and others
+// several (2 prompts of up to 32 tokens, 4 kv heads of 128: 11.5 us whole, 16
+// shared; of up to 48, half behind 256, fp8: 19 and 24); and `even`
+// batches (equal lengths, as many groups on every XCD) only lose the one L2 (16
+// prompts of 3740 at 2 kv heads of 128 497 and 523 us; 8 of 8192, 1073 and 1152).
+inline int shared_slots_log2(int n_y, int64_t num_seqs, int n_qtiles, bool even) {
   int l = 0;
   while (n_y << l < 8) ++l;
-  return n_y << l == 8 ? l : 0;
+  if (n_y << l != 8 || (n_y * num_seqs >= 8 && (n_qtiles < 2 << l || even))) return 0;
+  return l;
 }
 inline int64_t work_grid(int64_t n_x, int64_t U) { return U >= 8 ? 8 * ((U + 7) / 8) * n_x : U * n_x; }
 
@@ -1635,7 +1643,7 @@ struct RangePlan {
   static int64_t bytes() { return 2 * grid() * (kSlotO + kSlotL + static_cast<int64_t>(sizeof(int4))); }
   // Entries of a queue's list (an upper bound on what the kernel forms).
   static int64_t entries(int num_seqs, int n_qtiles, int n_y) {
-    const int rl = shared_slots_log2(n_y);
+    const int rl = shared_slots_log2(n_y, num_seqs, n_qtiles, false);
     const int64_t U = static_cast<int64_t>(n_y) * num_seqs;
     const int64_t w = rl > 0 ? 1 : (U >= 8 ? (n_y + 7) / 8 : n_y);
     return num_seqs * static_cast<int64_t>((n_qtiles + (1 << rl) - 1) >> rl) * w;
@@ -1664,7 +1672,7 @@ int launch_prefill_dma(PrefillArgs a, int64_t total_q, uint8_t *split_ws, int64_
   if (split_ws && split_bytes >= RP::bytes() &&
       RP::use(a.num_seqs, total_q, a.max_seqlen_q, a.max_seqlen_k, a.Hkv * a.quads, a.G4, FP8)) {
     const int grid = RP::grid();
-    a.rep_log2 = shared_slots_log2(a.Hkv * a.quads);
+    a.rep_log2 = shared_slots_log2(a.Hkv * a.quads, a.num_seqs, a.n_qtiles, false);
     if (a.rep_log2 > 0) a.pin = 1;
     a.part_o = reinterpret_cast<float *>(split_ws);
     a.part_l = reinterpret_cast<float *>(split_ws + 2 * grid * RP::kSlotO);
@@ -1688,7 +1696,9 @@ int launch_prefill_dma(PrefillArgs a, int64_t total_q, uint8_t *split_ws, int64_
   // (its groups x query tiles bound it), the (level, sequence) starts fit the
   // ring and the packed words hold the fields.
   const int64_t cx_max = U >= 8 ? (U + 7) / 8 : U;
-  const int rep_log2 = shared_slots_log2(a.Hkv * a.quads);
+  const bool even = U % 8 == 0 && total_q > 0 && 32 * total_q >= 31LL * a.num_seqs * a.max_seqlen_q &&
+                    8LL * a.max_seqlen_k <= 9LL * a.max_seqlen_q;
+  const int rep_log2 = shared_slots_log2(a.Hkv * a.quads, a.num_seqs, a.n_qtiles, even);
   if (rep_log2 > 0 &&
       static_cast<int64_t>(a.num_seqs) * ((a.n_qtiles + (1 << rep_log2) - 1) >> rep_log2) <= S::MAX_ITEMS)
     a.rep_log2 = rep_log2;

@@ -28,6 +28,35 @@ def test_prefill_shared_slots(cuda, hq, hkv, d):
         check(case, range(7), TOL_BF16, rows_per_seq=6, all_rows=True)
 
 
+@pytest.mark.parametrize("hkv,d", [(4, 128), (2, 128), (1, 128), (4, 256), (2, 256)])
+@pytest.mark.parametrize("lq", [1, 32, 33, 64, 257])
+def test_prefill_whole_groups(cuda, hkv, d, lq):
+    """8 groups or more of equal lengths, or of less than two query tiles per
+    XCD of a slot, stay whole: one tile, one over, and more tiles than that.  A
+    batch that shares its slots (one sequence shorter) gives the same bits for
+    the sequences they have in common."""
+    case = make_prefill_case("cfg3", seed=lq, device=cuda, nseq=8, lq=(lq, lq), prefix_blocks=(0, 0), hq=4 * hkv,
+                             hkv=hkv, d=d)
+    check(case, range(8), TOL_BF16, rows_per_seq=6, all_rows=True)
+    out = run_step(case)
+    n = 7 * lq
+    cu = case["cu_seqlens_q"].clone()
+    cu[8] = n + (lq + 1) // 2
+    q, k, v = (case[x][:int(cu[8])] for x in ("q", "k_new", "v_new"))
+    other = kernels.varlen_prefill(q, k, v, cu, cu, lq, lq, case["scale"])
+    assert torch.equal(other[:n], out[:n])
+
+
+@pytest.mark.parametrize("hkv,d", [(4, 128), (2, 128), (4, 256)])
+@pytest.mark.parametrize("kv", ["same", "fp8"])
+def test_prefill_ranges_whole_groups(cuda, hkv, d, kv):
+    """Ranges over 8 groups or more of one query tile each, behind prefixes of different lengths."""
+    case = make_prefill_case("cfg3", seed=9, device=cuda, nseq=8, lq=(1, 20), prefix_blocks=(2, 9), hq=4 * hkv, hkv=hkv,
+                             d=d, kv=kv)
+    assert _ranges(case)
+    check(case, range(8), TOL_FP8 if kv == "fp8" else TOL_BF16, rows_per_seq=8, all_rows=True)
+
+
 def _ranges(case):
     return lib().nq_prefill_split_workspace_bytes(case["nseq"], case["q"].shape[0], case["max_seqlen_q"],
                                                   case["max_seqlen_k"], case["hq"], case["hkv"], case["d"]) > 0

@@ -114,6 +114,8 @@ def test_ranges_cover_and_chain(n_y, rows, n_wg, tpb):
             lk[0] = max(0, lq[0] - 50)    # rows without any visible key
         pin = n_y * n >= 8
         rep = 8 // n_y if n_y < 8 and 8 % n_y == 0 else 1
+        if pin and cdiv(max(lq), rows) < 2 * rep:    # not enough query tiles to share
+            rep = 1
         pin = pin or rep > 1
         for x in range(8) if pin else (0,):
             check_queue(Queue(x, lq, lk, n_y, rows, pin, rep, n_wg if pin else 8 * n_wg, tpb, trial != 4))
