@@ -30,6 +30,7 @@ def _step(case, gate=None):
                                case["block_tables"], case["scale"], case["k_scale"], case["v_scale"], gate=gate,
                                k=case["k_new"], v=case["v_new"], slot_mapping=case["slot_mapping"])
     torch.cuda.synchronize()
+    assert kernels._key(case["q"].device) in kernels._decode_counters    # without a slot: two launches
     for pool in kernels._counter_pools.values():
         assert int(pool.count_nonzero()) == 0
     return out

@@ -8,10 +8,10 @@ import pytest
 import torch
 
 from nano_qwen_amd import kernels
-from nano_qwen_amd._lib import lib
 from oracle.inputs import make_prefill_case
 from tests.parity import TOL_BF16, TOL_FP8, assert_close, f64
 from tests.test_gpu_prefill import check, run_step
+from tests.test_prefill_ranges import would_cut
 
 pytestmark = pytest.mark.gpu
 
@@ -58,8 +58,10 @@ def test_prefill_ranges_whole_groups(cuda, hkv, d, kv):
 
 
 def _ranges(case):
-    return lib().nq_prefill_split_workspace_bytes(case["nseq"], case["q"].shape[0], case["max_seqlen_q"],
-                                                  case["max_seqlen_k"], case["hq"], case["hkv"], case["d"]) > 0
+    """Whether the library cuts the case's launch (as tests/test_prefill_ranges.py asks it)."""
+    kv = case["k_cache"].dtype if case["block_tables"] is not None else case["k_new"].dtype
+    return would_cut(case["nseq"], case["q"].shape[0], case["max_seqlen_q"], case["max_seqlen_k"], case["hq"],
+                     case["hkv"], case["d"], kv)
 
 
 @pytest.mark.parametrize("kw", [

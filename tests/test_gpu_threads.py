@@ -8,14 +8,15 @@ import torch
 
 from nano_qwen_amd import kernels
 from oracle.inputs import make_decode_case, make_prefill_case
+from tests.test_prefill_ranges import would_cut
 
 pytestmark = pytest.mark.gpu
 
 
 def _prefill(device, i):
     c = make_prefill_case("cfg3", seed=i, device=device, nseq=2, lq=(90, 300), prefix_blocks=(3, 8))
-    assert kernels.lib().nq_prefill_split_workspace_bytes(c["nseq"], c["q"].shape[0], c["max_seqlen_q"],
-                                                          c["max_seqlen_k"], c["hq"], c["hkv"], c["d"]) > 0
+    assert would_cut(2, c["q"].shape[0], c["max_seqlen_q"], c["max_seqlen_k"], c["hq"], c["hkv"], c["d"],
+                     c["k_cache"].dtype)
     kernels.store_kvcache(c["k_new"], c["v_new"], c["k_cache"], c["v_cache"], c["slot_mapping"])
     return lambda: kernels.varlen_prefill(c["q"], c["k_cache"], c["v_cache"], c["cu_seqlens_q"], c["cu_seqlens_k"],
                                           c["max_seqlen_q"], c["max_seqlen_k"], c["scale"],

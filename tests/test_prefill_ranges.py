@@ -121,7 +121,7 @@ def test_ranges_cover_and_chain(n_y, rows, n_wg, tpb):
             check_queue(Queue(x, lq, lk, n_y, rows, pin, rep, n_wg if pin else 8 * n_wg, tpb, trial != 4))
 
 
-def _cut(n, total_q, max_q, max_k, hq, hkv, d, kv):
+def would_cut(n, total_q, max_q, max_k, hq, hkv, d, kv):
     """Whether the library would cut such a launch: it asks for the partials' buffer, with nothing launched."""
     need = ctypes.c_int64()
     rc = lib().nq_varlen_prefill_split(None, 0, 0, None, None, 0, None, None, max_q, max_k, None, 0, 0, 0, None, 0, 0, n,
@@ -150,4 +150,4 @@ BF16, FP8 = torch.bfloat16, torch.float8_e4m3fn
 def test_which_launches_are_cut(n, total_q, max_q, prefix, d, kv, cut):
     hq, hkv = (16, 4) if d == 256 else (32, 8)
     hkv = 2 if n == 12 else hkv
-    assert _cut(n, total_q, max_q, max_q + prefix, 4 * hkv, hkv, d, kv) == cut
+    assert would_cut(n, total_q, max_q, max_q + prefix, 4 * hkv, hkv, d, kv) == cut
