@@ -60,10 +60,11 @@
 //      without values, which gives M;
 //   2. gdn_combine_kernel chains them, in float32 throughout (fp32 MFMA);
 //   3. gdn_chunk_kernel<kSegment> runs every segment from the state it enters with.
-// Three times the work of the chain, in parallel over all segments.  Chunks
+// A chunk runs up to three times, twice of them for its state only: about two
+// and a half times the chain's work, in parallel over all segments.  Chunks
 // start where they do without segments; the states and outputs differ from
-// the chain's as two float32 summation orders do (errors against float64 are
-// the same within 3%).
+// the chain's as two float32 summation orders do, and agree where the decay
+// forgets a segment's start (errors against float64 are the same within 3%).
 #include <algorithm>
 
 #include "nq_device.hpp"

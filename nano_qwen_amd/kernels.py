@@ -80,12 +80,13 @@ def _grow(table, key, nbytes, dtype, device, zero=False):
 
 
 def release_workspaces(device=None) -> int:
-    """Drop the kernels' per-stream buffers (decode split-K workspaces,
-    prefill queue counters and partial outputs, GDN segment states) and every retired buffer, of ``device`` or of
-    all devices; returns how many were dropped.  Only safe once no HIP graph
-    captured with them will be replayed again: a replay would write freed
-    memory.  Later calls allocate fresh buffers (the prefill counters start
-    at zero again)."""
+    """Drop the kernels' per-stream buffers (decode split-K workspaces and
+    arrival counters, prefill queue counters and partial outputs, GDN segment
+    states) and every retired buffer, of ``device`` or of all devices; returns
+    how many were dropped.  Only safe once no HIP graph captured with them will
+    be replayed again (a replay would write freed memory) and while no other
+    thread calls the kernels.  Later calls allocate fresh buffers (the counters
+    start at zero again)."""
     idx = None if device is None else _key(device)[0]
     n = 0
     for table in (_workspaces, _prefill_queues, _prefill_parts, _gdn_segments, _decode_counters,
@@ -358,8 +359,7 @@ def varlen_prefill(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen
     Without ``block_table``: ``k, v [Tk, Hkv, D]`` packed by ``cu_seqlens_k``.
     With it: ``k, v`` are the paged caches ``[num_blocks, block_size, Hkv, D]``.
     With ``gate [Tq, Hq, D]`` the output is ``out * sigmoid(gate)``
-    (models/qwen3_5.py:142), applied in the kernel's output store (16-bit
-    K/V) or by one in-place pass after it (fp8 K/V).
+    (models/qwen3_5.py:142), applied in the kernel's output store.
     """
     require_cuda(q, k, v, cu_seqlens_q, cu_seqlens_k, block_table, what="varlen_prefill")
     tq, hq, d = q.shape
