@@ -57,8 +57,9 @@ def _launch_lock(key: tuple[int, int]):
 
 
 def _key(device) -> tuple[int, int]:
-    dev = torch.device(device)
-    idx = dev.index if dev.index is not None else torch.cuda.current_device()
+    idx = (device if isinstance(device, torch.device) else torch.device(device)).index
+    if idx is None:
+        idx = torch.cuda.current_device()
     return idx, raw_stream(idx)
 
 
@@ -217,7 +218,7 @@ def _decode_counter_slot(key: tuple[int, int]) -> torch.Tensor | None:
     have a slot of their own, and a capture's first decode records its zeroing,
     so that the damage ends with those replays.  Called with the stream's
     launch lock held."""
-    if not torch.cuda.is_current_stream_capturing():
+    if key[1] == 0 or not torch.cuda.is_current_stream_capturing():    # the null stream cannot be captured
         slot = _decode_counters.get(key)
         return slot if slot is not None else _take_counter_slot(key, False)
     last, slot = _capture_counters.get(key, (0, None))
