@@ -218,10 +218,11 @@ int nq_paged_decode_store(const void *q, int64_t q_batch_stride, int64_t q_head_
  * bytes of device memory per (sequence, kv head), 64-byte aligned, zero before
  * the first call that uses them; every completed call leaves them zero.  Calls
  * that overlap may share neither them nor the workspace: counters that an overlap
- * left nonzero spoil the calls after it too.  A capture had better zero its
- * counters ahead of its first call (nq_capture_id tells a new capture), so that
- * replays that overlapped spoil no later one.  num_splits and split_tokens as
- * nq_decode_config gives them (any plan that nq_paged_decode accepts is).
+ * left nonzero spoil the calls after it too.  A capture had better have counters
+ * of its own, or zero them ahead of its first call (nq_capture_id tells a new
+ * capture), so that replays that overlapped spoil no later one.  num_splits and
+ * split_tokens as nq_decode_config gives them (any plan that nq_paged_decode
+ * accepts is).
  */
 int nq_paged_decode_fused(const void *q, int64_t q_batch_stride, int64_t q_head_stride,
                           void *k_cache, void *v_cache, const int32_t *block_tables, int64_t bt_stride,

@@ -38,13 +38,15 @@ _prefill_queues: dict[tuple[int, int], torch.Tensor] = {}
 _prefill_parts: dict[tuple[int, int], torch.Tensor] = {}
 _gdn_segments: dict[tuple[int, int], torch.Tensor] = {}
 _retired: list[torch.Tensor] = []
-# Zeroed arrival counters of the one-launch decode: a pool per device, a slot
-# per (device, stream) and a second one for what is captured on that stream,
-# with the id of the last capture that zeroed it.
-_COUNTER_SLOTS, _COUNTER_SLOT_BYTES = 64, 128 << 10
+# Zeroed arrival counters of the one-launch decode: a pool per device; of its
+# slots one kind is for streams (_decode_counters, and _shared_counters for
+# captures that found none of their own), the other for one capture each.
+_COUNTER_SLOTS, _COUNTER_SLOT_BYTES = 64, 128 << 10    # slots of each kind
 _counter_pools: dict[int, torch.Tensor] = {}
+_counter_slots_taken: dict[tuple[int, int], int] = {}    # (device, kind)
 _decode_counters: dict[tuple[int, int], torch.Tensor] = {}
-_capture_counters: dict[tuple[int, int], tuple[int, torch.Tensor]] = {}
+_shared_counters: dict[tuple[int, int], torch.Tensor] = {}
+_capture_counters: dict[tuple[int, int], tuple[int, torch.Tensor | None]] = {}    # last capture's id and slot
 _counter_lock = threading.Lock()
 # A fixed set of locks, so that streams come and go without leaving any (two
 # streams that share one only wait for each other's host calls).
@@ -91,12 +93,14 @@ def release_workspaces(device=None) -> int:
     idx = None if device is None else _key(device)[0]
     n = 0
     for table in (_workspaces, _prefill_queues, _prefill_parts, _gdn_segments, _decode_counters,
-                  _capture_counters):
+                  _shared_counters, _capture_counters):
         for key in [k for k in table if idx is None or k[0] == idx]:
             del table[key]
             n += 1
     for dev in [k for k in _counter_pools if idx is None or k == idx]:
         del _counter_pools[dev]
+        _counter_slots_taken.pop((dev, 0), None)
+        _counter_slots_taken.pop((dev, 1), None)
     keep = [t for t in _retired if idx is not None and t.device.index != idx]
     n += len(_retired) - len(keep)
     _retired[:] = keep
@@ -134,6 +138,14 @@ def decode_plan(batch, num_q_heads, num_kv_heads, max_blocks_per_seq, block_size
                               dtype_code(kv_dtype), ctypes.byref(ns), ctypes.byref(st))
     check(rc, "decode_plan")
     return ns.value, st.value
+
+
+def _decode_config(batch, num_q_heads, num_kv_heads, head_dim, max_blocks_per_seq, block_size, kv_dtype):
+    """nq_decode_config: bytes of counters (0: two launches), splits, their tokens, bytes of workspace."""
+    config = (ctypes.c_int64 * 4)()
+    check(lib().nq_decode_config(batch, num_q_heads, num_kv_heads, head_dim, max_blocks_per_seq, block_size,
+                                 dtype_code(kv_dtype), config), "decode_config")
+    return config
 
 
 def decode_schedule(batch, num_q_heads, num_kv_heads, head_dim, max_blocks_per_seq, block_size, kv_dtype,
@@ -175,61 +187,73 @@ def reserve_decode_workspace(device, max_batch, num_q_heads, num_kv_heads, max_b
     for b in range(1, int(max_batch) + 1):
         ns, _ = decode_plan(b, num_q_heads, num_kv_heads, max_blocks_per_seq, block_size, kv_dtype)
         need = max(need, lib().nq_decode_workspace_bytes(b, num_q_heads, head_dim, ns))
-        config = (ctypes.c_int64 * 4)()    # the one-launch path's own plan
-        check(lib().nq_decode_config(b, num_q_heads, num_kv_heads, head_dim, max_blocks_per_seq, block_size,
-                                     dtype_code(kv_dtype), config), "decode_config")
-        need = max(need, config[3])
+        config = _decode_config(b, num_q_heads, num_kv_heads, head_dim, max_blocks_per_seq, block_size, kv_dtype)
+        need = max(need, config[3])    # the one-launch path's own plan
     if need > 0:
         decode_workspace(device, need)
     return need
 
 
-def _take_counter_slot(key: tuple[int, int], capturing: bool) -> torch.Tensor | None:
+def _take_counter_slot(key: tuple[int, int], kind: int, capturing: bool) -> torch.Tensor | None:
     """A slot of the device's pool, which is zeroed and waited for when it is
-    made.  ``None`` -- the decode then takes its two-launch path -- when the pool
-    would have to be made during a capture or has no slot left."""
+    made.  ``None`` when the pool would have to be made during a capture or has
+    no slot of that kind left."""
     with _counter_lock:
         pool = _counter_pools.get(key[0])
         if pool is None:
             if capturing:
                 return None
-            pool = torch.zeros(_COUNTER_SLOTS, _COUNTER_SLOT_BYTES // 4, dtype=torch.int32,
+            pool = torch.zeros(2 * _COUNTER_SLOTS, _COUNTER_SLOT_BYTES // 4, dtype=torch.int32,
                                device=torch.device("cuda", key[0]))
             torch.cuda.current_stream(key[0]).synchronize()
             _counter_pools[key[0]] = pool
-        used = sum(k[0] == key[0] for table in (_decode_counters, _capture_counters) for k in table)
+        used = _counter_slots_taken.get((key[0], kind), 0)
         if used >= _COUNTER_SLOTS:
             return None
+        _counter_slots_taken[key[0], kind] = used + 1
         # the pool was made on another stream: released, it is not handed
         # out again before this stream's launches have ended
         pool.record_stream(torch.cuda.current_stream(key[0]))
-        if capturing:
-            _capture_counters[key] = 0, pool[used]
-        else:
-            _decode_counters[key] = pool[used]
-        return pool[used]
+        return pool[used + kind * _COUNTER_SLOTS]
+
+
+def _capturing(key: tuple[int, int]) -> bool:
+    return key[1] != 0 and torch.cuda.is_current_stream_capturing()    # the null stream cannot be captured
 
 
 def _decode_counter_slot(key: tuple[int, int]) -> torch.Tensor | None:
-    """Arrival counters of the one-launch decode for a (device, stream).  Every
-    launch leaves its counters zero again, so those of a stream's own launches
-    stay in order.  Graphs captured on one stream may be replayed on several,
-    and replays that overlap spoil their common counters: captured launches
-    have a slot of their own, and a capture's first decode records its zeroing,
-    so that the damage ends with those replays.  Called with the stream's
-    launch lock held."""
-    if key[1] == 0 or not torch.cuda.is_current_stream_capturing():    # the null stream cannot be captured
-        slot = _decode_counters.get(key)
-        return slot if slot is not None else _take_counter_slot(key, False)
-    last, slot = _capture_counters.get(key, (0, None))
+    """Arrival counters of the one-launch decode for a (device, stream): every
+    launch leaves its counters zero again, and a stream's launches are in order.
+    ``None`` (no slot left): the decode takes two launches.  Called with the
+    stream's launch lock held, as the next."""
+    slot = _decode_counters.get(key)
     if slot is None:
-        slot = _take_counter_slot(key, True)
-        if slot is None:
-            return None
+        slot = _take_counter_slot(key, 0, False)
+        if slot is not None:
+            _decode_counters[key] = slot
+    return slot
+
+
+def _captured_counter_slot(key: tuple[int, int]) -> torch.Tensor | None:
+    """The same for a stream that is being captured.  Graphs captured on one
+    stream may be replayed on several, and replays that overlap would spoil
+    common counters for good: every capture takes a slot of its own.  Captures
+    past the pool's slots share one per stream, whose zeroing the first decode
+    of each records (a node of its own in every replay, about 2 us), so that the
+    damage ends with the replays that overlapped."""
+    last, slot = _capture_counters.get(key, (0, None))
     now = lib().nq_capture_id(key[1])
-    if now != last or now == 0:
-        slot.zero_()    # a fill kernel
-        _capture_counters[key] = now, slot
+    if now == last != 0:
+        return slot
+    slot = _take_counter_slot(key, 1, True) if now != 0 else None
+    if slot is None:
+        slot = _shared_counters.get(key)
+        if slot is None:
+            slot = _take_counter_slot(key, 0, True)
+        if slot is not None:
+            _shared_counters[key] = slot
+            slot.zero_()    # a fill kernel
+    _capture_counters[key] = now, slot
     return slot
 
 
@@ -323,7 +347,12 @@ def paged_decode(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale,
     key = _key(q.device)
     need = ctypes.c_int64()
     with _launch_lock(key):
-        counters = _decode_counter_slot(key)
+        if not _capturing(key):
+            counters = _decode_counter_slot(key)
+        elif _decode_config(B, hq, hkv, d, block_table.shape[1], bs, kv_dtype)[0] > 0:
+            counters = _captured_counter_slot(key)
+        else:
+            counters = None
         ws = _workspaces.get(key)
         while True:
             rc = lib().nq_paged_decode_auto(

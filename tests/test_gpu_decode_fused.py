@@ -116,33 +116,68 @@ def test_fused_decode_streams_have_their_own_counters(cuda):
     assert slots[0] != slots[1]
 
 
-def test_fused_decode_spoiled_counters_do_not_last(cuda):
-    """Counters that an overlap of two replays left nonzero (every slot of the
-    pool but the eager stream's): the graphs' next replays are right, and leave
-    theirs zero."""
-    cases = [make_decode_case("cfg2", seed=s, device=cuda, batch=2, ctx=(700, 700), hq=8, hkv=2) for s in (5, 6)]
+def _capture_two(device):
+    """Two graphs on torch's own capture stream, as two runners capture, of
+    three decodes each: (arguments, graphs, outputs, eager results)."""
+    cases = [make_decode_case("cfg2", seed=s, device=device, batch=2, ctx=(700, 700), hq=8, hkv=2) for s in (5, 6)]
+    assert all(map(_fused, cases))
     args = [(c["q"].unsqueeze(1), c["k_cache"], c["v_cache"], c["context_lens"], c["block_tables"], c["scale"])
             for c in cases]
-    assert all(map(_fused, cases))
     want = [kernels.paged_decode(*a) for a in args]
     torch.cuda.synchronize()
-    graphs, outs = [], []
-    for a in args:    # as a runner captures: torch's own capture stream, several decodes each
+    graphs, outs, slots = [], [], []
+    for a in args:
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph):
             outs.append([kernels.paged_decode(*a) for _ in range(3)])
+            slots.append(kernels._capture_counters[kernels._key(device)][1])
         graphs.append(graph)
+    return args, graphs, outs, want, slots
+
+
+def _replay(graph, got, want):
+    for o in got:
+        o.zero_()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, want) for o in got)
+
+
+def test_fused_decode_captures_have_their_own_counters(cuda):
+    """Spoiled counters of anything else -- every slot of the pool but the graph's
+    own, as overlapping replays leave them -- do not reach a graph's replays."""
+    args, graphs, outs, want, slots = _capture_two(cuda)
     pool = kernels._counter_pools[0]
-    eager = kernels._decode_counters[(0, torch.cuda.current_stream().cuda_stream)]
+    eager = kernels._decode_counters[kernels._key(cuda)]
+    assert len({t.data_ptr() for t in (*slots, eager)}) == 3
+    for _ in range(3):
+        for graph, got, w, slot in zip(graphs, outs, want, slots):
+            pool.fill_(7)
+            slot.zero_()
+            _replay(graph, got, w)
+            assert not slot.any()
+    pool.zero_()
+    for _ in range(3):
+        for graph, got, w in zip(graphs, outs, want):
+            _replay(graph, got, w)
+            assert torch.equal(kernels.paged_decode(*args[0]), want[0])
+    assert not pool.any()
+
+
+def test_fused_decode_spoiled_counters_do_not_last(cuda, monkeypatch):
+    """Captures past the pool's slots share one: what an overlap leaves in it (here
+    in every slot but the eager stream's) ends with the next replay."""
+    kernels._take_counter_slot(kernels._key(cuda), 0, False)    # the pool is there
+    monkeypatch.setitem(kernels._counter_slots_taken, (0, 1), kernels._COUNTER_SLOTS)
+    args, graphs, outs, want, slots = _capture_two(cuda)
+    assert slots[0].data_ptr() == slots[1].data_ptr()
+    pool = kernels._counter_pools[0]
+    eager = kernels._decode_counters[kernels._key(cuda)]
     for _ in range(3):
         for graph, got, w in zip(graphs, outs, want):
             pool.fill_(7)
             eager.zero_()
-            for o in got:
-                o.zero_()
-            graph.replay()
-            torch.cuda.synchronize()
-            assert all(torch.equal(o, w) for o in got)
+            _replay(graph, got, w)
             assert torch.equal(kernels.paged_decode(*args[0]), want[0])
     pool.zero_()
     torch.cuda.synchronize()

@@ -68,6 +68,7 @@ def library(monkeypatch):
     monkeypatch.setattr(kernels, "lib", lambda: fake)
     monkeypatch.setattr(kernels, "require_cuda", lambda *a, **k: None)
     monkeypatch.setattr(kernels, "_key", lambda device: (0, getattr(stream, "handle", 0)))
+    monkeypatch.setattr(kernels, "_capturing", lambda key: False)
     monkeypatch.setattr(kernels, "_decode_counter_slot", lambda key: None)
     for table in ("_workspaces", "_prefill_queues", "_prefill_parts", "_gdn_segments"):
         monkeypatch.setattr(kernels, table, {})
