@@ -38,12 +38,12 @@ _prefill_queues: dict[tuple[int, int], torch.Tensor] = {}
 _prefill_parts: dict[tuple[int, int], torch.Tensor] = {}
 _gdn_segments: dict[tuple[int, int], torch.Tensor] = {}
 _retired: list[torch.Tensor] = []
-# Zeroed arrival counters of the one-launch decode: a pool per device; of its
-# slots one kind is for streams (_decode_counters, and _shared_counters for
-# captures that found none of their own), the other for one capture each.
-_COUNTER_SLOTS, _COUNTER_SLOT_BYTES = 64, 128 << 10    # slots of each kind
+# Zeroed arrival counters of the one-launch decode: a pool per device, one half
+# for streams (_decode_counters, and _shared_counters for captures that found no
+# room in the other), one for captures, each handed out from its start.
+_COUNTER_SLOT_BYTES, _COUNTER_HALF_BYTES = 128 << 10, 8 << 20
 _counter_pools: dict[int, torch.Tensor] = {}
-_counter_slots_taken: dict[tuple[int, int], int] = {}    # (device, kind)
+_counter_bytes_taken: dict[tuple[int, int], int] = {}    # (device, half)
 _decode_counters: dict[tuple[int, int], torch.Tensor] = {}
 _shared_counters: dict[tuple[int, int], torch.Tensor] = {}
 _capture_counters: dict[tuple[int, int], tuple[int, torch.Tensor | None]] = {}    # last capture's id and slot
@@ -99,8 +99,8 @@ def release_workspaces(device=None) -> int:
             n += 1
     for dev in [k for k in _counter_pools if idx is None or k == idx]:
         del _counter_pools[dev]
-        _counter_slots_taken.pop((dev, 0), None)
-        _counter_slots_taken.pop((dev, 1), None)
+        _counter_bytes_taken.pop((dev, 0), None)
+        _counter_bytes_taken.pop((dev, 1), None)
     keep = [t for t in _retired if idx is not None and t.device.index != idx]
     n += len(_retired) - len(keep)
     _retired[:] = keep
@@ -194,27 +194,26 @@ def reserve_decode_workspace(device, max_batch, num_q_heads, num_kv_heads, max_b
     return need
 
 
-def _take_counter_slot(key: tuple[int, int], kind: int, capturing: bool) -> torch.Tensor | None:
-    """A slot of the device's pool, which is zeroed and waited for when it is
-    made.  ``None`` when the pool would have to be made during a capture or has
-    no slot of that kind left."""
+def _take_counter_slot(key: tuple[int, int], half: int, nbytes: int, capturing: bool) -> torch.Tensor | None:
+    """Counters from a half of the device's pool, which is zeroed and waited for
+    when it is made.  ``None`` when the pool would have to be made during a
+    capture or the half has no room left."""
     with _counter_lock:
         pool = _counter_pools.get(key[0])
         if pool is None:
             if capturing:
                 return None
-            pool = torch.zeros(2 * _COUNTER_SLOTS, _COUNTER_SLOT_BYTES // 4, dtype=torch.int32,
-                               device=torch.device("cuda", key[0]))
+            pool = torch.zeros(2, _COUNTER_HALF_BYTES // 4, dtype=torch.int32, device=torch.device("cuda", key[0]))
             torch.cuda.current_stream(key[0]).synchronize()
             _counter_pools[key[0]] = pool
-        used = _counter_slots_taken.get((key[0], kind), 0)
-        if used >= _COUNTER_SLOTS:
+        used = _counter_bytes_taken.get((key[0], half), 0)
+        if used + nbytes > _COUNTER_HALF_BYTES:
             return None
-        _counter_slots_taken[key[0], kind] = used + 1
+        _counter_bytes_taken[key[0], half] = used + nbytes
         # the pool was made on another stream: released, it is not handed
         # out again before this stream's launches have ended
         pool.record_stream(torch.cuda.current_stream(key[0]))
-        return pool[used + kind * _COUNTER_SLOTS]
+        return pool[half, used // 4:(used + nbytes) // 4]
 
 
 def _capturing(key: tuple[int, int]) -> bool:
@@ -228,28 +227,29 @@ def _decode_counter_slot(key: tuple[int, int]) -> torch.Tensor | None:
     stream's launch lock held, as the next."""
     slot = _decode_counters.get(key)
     if slot is None:
-        slot = _take_counter_slot(key, 0, False)
+        slot = _take_counter_slot(key, 0, _COUNTER_SLOT_BYTES, False)
         if slot is not None:
             _decode_counters[key] = slot
     return slot
 
 
-def _captured_counter_slot(key: tuple[int, int]) -> torch.Tensor | None:
-    """The same for a stream that is being captured.  Graphs captured on one
-    stream may be replayed on several, and replays that overlap would spoil
-    common counters for good: every capture takes a slot of its own.  Captures
-    past the pool's slots share one per stream, whose zeroing the first decode
-    of each records (a node of its own in every replay, about 2 us), so that the
-    damage ends with the replays that overlapped."""
+def _captured_counter_slot(key: tuple[int, int], nbytes: int) -> torch.Tensor | None:
+    """The same for a decode that needs ``nbytes`` of them on a stream that is
+    being captured.  Graphs captured on one stream may be replayed on several,
+    and replays that overlap would spoil common counters for good: every capture
+    has its own, of its largest decode's size in steps of 4 KiB.  Captures that
+    find no room share a slot per stream, whose zeroing each records (a node of
+    its own in every replay, about 4 us), so that the damage ends with the
+    replays that overlapped."""
     last, slot = _capture_counters.get(key, (0, None))
     now = lib().nq_capture_id(key[1])
-    if now == last != 0:
+    if now == last != 0 and (slot is None or slot.numel() * 4 >= nbytes):
         return slot
-    slot = _take_counter_slot(key, 1, True) if now != 0 else None
+    slot = _take_counter_slot(key, 1, -(-nbytes // 4096) * 4096, True) if now != 0 else None
     if slot is None:
         slot = _shared_counters.get(key)
         if slot is None:
-            slot = _take_counter_slot(key, 0, True)
+            slot = _take_counter_slot(key, 0, _COUNTER_SLOT_BYTES, True)
         if slot is not None:
             _shared_counters[key] = slot
             slot.zero_()    # a fill kernel
@@ -349,10 +349,9 @@ def paged_decode(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale,
     with _launch_lock(key):
         if not _capturing(key):
             counters = _decode_counter_slot(key)
-        elif _decode_config(B, hq, hkv, d, block_table.shape[1], bs, kv_dtype)[0] > 0:
-            counters = _captured_counter_slot(key)
         else:
-            counters = None
+            nbytes = _decode_config(B, hq, hkv, d, block_table.shape[1], bs, kv_dtype)[0]
+            counters = _captured_counter_slot(key, nbytes) if 0 < nbytes <= _COUNTER_SLOT_BYTES else None
         ws = _workspaces.get(key)
         while True:
             rc = lib().nq_paged_decode_auto(
@@ -361,7 +360,7 @@ def paged_decode(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale,
                 B, hq, hkv, d, bs, nb, float(softmax_scale), ptr(ws), 0 if ws is None else ws.numel(),
                 dtype_code(q.dtype), dtype_code(kv_dtype), ptr(k_scale) if fp8 else None,
                 ptr(v_scale) if fp8 else None, g_ptr, g_bs, g_hs, ptr(counters),
-                0 if counters is None else _COUNTER_SLOT_BYTES, need, key[1])
+                0 if counters is None else counters.numel() * 4, need, key[1])
             if rc != 1:
                 break
             ws = decode_workspace(q.device, need.value)

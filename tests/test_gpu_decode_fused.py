@@ -164,11 +164,36 @@ def test_fused_decode_captures_have_their_own_counters(cuda):
     assert not pool.any()
 
 
+def test_fused_decode_counters_of_a_larger_decode(cuda):
+    """A capture whose second decode is larger takes counters for it, too."""
+    small, large = (make_decode_case("cfg2", seed=s, device=cuda, batch=b, ctx=(400, 400), hq=8, hkv=2)
+                    for s, b in ((7, 1), (8, 200)))
+    args = [(c["q"].unsqueeze(1), c["k_cache"], c["v_cache"], c["context_lens"], c["block_tables"], c["scale"])
+            for c in (small, large)]
+    assert _fused(small) and _fused(large)
+    want = [kernels.paged_decode(*a) for a in args]
+    graph = torch.cuda.CUDAGraph()
+    key = []
+    with torch.cuda.graph(graph):
+        outs = []
+        for i in (0, 1, 0):
+            outs.append(kernels.paged_decode(*args[i]))
+            key.append(kernels._capture_counters[kernels._key(cuda)][1])
+    assert key[0].numel() * 4 == 4096 and key[1].numel() * 4 == 28 << 10 and key[2] is key[1]
+    for _ in range(3):
+        for o in outs:
+            o.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, want[i]) for o, i in zip(outs, (0, 1, 0)))
+    assert not kernels._counter_pools[0].any()
+
+
 def test_fused_decode_spoiled_counters_do_not_last(cuda, monkeypatch):
-    """Captures past the pool's slots share one: what an overlap leaves in it (here
+    """Captures that find no room in the pool share a slot: what an overlap leaves in it (here
     in every slot but the eager stream's) ends with the next replay."""
-    kernels._take_counter_slot(kernels._key(cuda), 0, False)    # the pool is there
-    monkeypatch.setitem(kernels._counter_slots_taken, (0, 1), kernels._COUNTER_SLOTS)
+    kernels._take_counter_slot(kernels._key(cuda), 0, 4096, False)    # the pool is there
+    monkeypatch.setitem(kernels._counter_bytes_taken, (0, 1), kernels._COUNTER_HALF_BYTES)
     args, graphs, outs, want, slots = _capture_two(cuda)
     assert slots[0].data_ptr() == slots[1].data_ptr()
     pool = kernels._counter_pools[0]
