@@ -55,7 +55,7 @@ _DEBUG_QUEUE = os.environ.get("NQ_DEBUG_PREFILL_QUEUE", "0") not in ("", "0")
 
 
 def _launch_lock(key: tuple[int, int]):
-    return _launch_locks[hash(key) % len(_launch_locks)]
+    return _launch_locks[hash(key) & 63]
 
 
 def _key(device) -> tuple[int, int]:
@@ -217,19 +217,17 @@ def _take_counter_slot(key: tuple[int, int], half: int, nbytes: int, capturing: 
 
 
 def _capturing(key: tuple[int, int]) -> bool:
-    return key[1] != 0 and torch.cuda.is_current_stream_capturing()    # the null stream cannot be captured
+    return torch.cuda.is_current_stream_capturing()
 
 
 def _decode_counter_slot(key: tuple[int, int]) -> torch.Tensor | None:
-    """Arrival counters of the one-launch decode for a (device, stream): every
-    launch leaves its counters zero again, and a stream's launches are in order.
-    ``None`` (no slot left): the decode takes two launches.  Called with the
-    stream's launch lock held, as the next."""
-    slot = _decode_counters.get(key)
-    if slot is None:
-        slot = _take_counter_slot(key, 0, _COUNTER_SLOT_BYTES, False)
-        if slot is not None:
-            _decode_counters[key] = slot
+    """Arrival counters of the one-launch decode for a (device, stream) that has
+    none: every launch leaves its counters zero again, and a stream's launches
+    are in order.  ``None`` (no slot left): the decode takes two launches.
+    Called with the stream's launch lock held, as the next."""
+    slot = _take_counter_slot(key, 0, _COUNTER_SLOT_BYTES, False)
+    if slot is not None:
+        _decode_counters[key] = slot
     return slot
 
 
@@ -346,12 +344,14 @@ def paged_decode(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale,
     # The library picks the plan; it asks for a larger workspace once.
     key = _key(q.device)
     need = ctypes.c_int64()
-    with _launch_lock(key):
-        if not _capturing(key):
-            counters = _decode_counter_slot(key)
-        else:
+    with _launch_locks[hash(key) & 63]:
+        if key[1] != 0 and _capturing(key):    # the null stream cannot be captured
             nbytes = _decode_config(B, hq, hkv, d, block_table.shape[1], bs, kv_dtype)[0]
             counters = _captured_counter_slot(key, nbytes) if 0 < nbytes <= _COUNTER_SLOT_BYTES else None
+        else:
+            counters = _decode_counters.get(key)
+            if counters is None:
+                counters = _decode_counter_slot(key)
         ws = _workspaces.get(key)
         while True:
             rc = lib().nq_paged_decode_auto(
