@@ -250,7 +250,8 @@ def _captured_counter_slot(key: tuple[int, int], nbytes: int) -> torch.Tensor | 
             slot = _take_counter_slot(key, 0, _COUNTER_SLOT_BYTES, True)
         if slot is not None:
             _shared_counters[key] = slot
-            slot.zero_()    # a fill kernel
+            with torch.inference_mode():    # the pool may have been made there, or not
+                slot.zero_()    # a fill kernel
     _capture_counters[key] = now, slot
     return slot
 

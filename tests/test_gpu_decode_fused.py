@@ -192,7 +192,9 @@ def test_fused_decode_counters_of_a_larger_decode(cuda):
 def test_fused_decode_spoiled_counters_do_not_last(cuda, monkeypatch):
     """Captures that find no room in the pool share a slot: what an overlap leaves in it (here
     in every slot but the eager stream's) ends with the next replay."""
-    kernels._take_counter_slot(kernels._key(cuda), 0, 4096, False)    # the pool is there
+    kernels.release_workspaces()
+    with torch.inference_mode():    # a pool made there is used outside, too
+        kernels._take_counter_slot(kernels._key(cuda), 0, 4096, False)
     monkeypatch.setitem(kernels._counter_bytes_taken, (0, 1), kernels._COUNTER_HALF_BYTES)
     args, graphs, outs, want, slots = _capture_two(cuda)
     assert slots[0].data_ptr() == slots[1].data_ptr()
@@ -200,11 +202,12 @@ def test_fused_decode_spoiled_counters_do_not_last(cuda, monkeypatch):
     eager = kernels._decode_counters[kernels._key(cuda)]
     for _ in range(3):
         for graph, got, w in zip(graphs, outs, want):
-            pool.fill_(7)
-            eager.zero_()
+            with torch.inference_mode():
+                pool.fill_(7)
+                eager.zero_()
             _replay(graph, got, w)
             assert torch.equal(kernels.paged_decode(*args[0]), want[0])
-    pool.zero_()
+    kernels.release_workspaces()
     torch.cuda.synchronize()
 
 
